@@ -367,6 +367,32 @@ __device__ __forceinline__ void load_spinor(vec2<R> (&s)[12], const vec2<R>* __r
         }
     }
 }
+/* the spinors of N site offsets, 16-byte lane by 16-byte lane: lane q of every one of them before lane q + 1
+ * (for two spinors a compiler barrier holds that order) */
+template<typename R, int N>
+__device__ __forceinline__ void load_spinors_interleaved(vec2<R> (&s)[N][12], const vec2<R>* __restrict__ in, size_t CS,
+                                                         const size_t (&o)[N])
+{
+    if constexpr (sizeof(R) == 8) {
+#pragma unroll
+        for (int k = 0; k < 12; ++k) {
+#pragma unroll
+            for (int n = 0; n < N; ++n) s[n][k] = in[(size_t)k * CS + o[n]];
+        }
+    } else {
+        const float4* p = reinterpret_cast<const float4*>(in);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+#pragma unroll
+            for (int n = 0; n < N; ++n) {
+                const float4 v  = p[(size_t)q * CS + o[n]];
+                s[n][2 * q]     = vec2<R>{v.x, v.y};
+                s[n][2 * q + 1] = vec2<R>{v.z, v.w};
+            }
+            if constexpr (N == 2) asm volatile("" ::: "memory");
+        }
+    }
+}
 /* the same with streaming loads (data read once) */
 template<typename R>
 __device__ __forceinline__ void load_spinor_stream(vec2<R> (&s)[12], const vec2<R>* in, size_t CS, size_t o)

@@ -69,27 +69,51 @@ __device__ __forceinline__ void apply_hop(Cx<R> (&acc)[12], const vec2<R> (&s)[1
 /* forward and backward hop of direction DIR: both links and both neighbour spinors (elements nf, nbk
  * of the spinor field) are loaded before either hop is applied.  The forward link is the output
  * site's own (eo index i, parity P), the backward one the neighbour's (eo index linkbk, parity P^1). */
-/* forward and backward hops of directions D0 and D1: four links and four neighbour spinors in flight
- * before any hop is applied (the 1-wave-per-SIMD variants, which may also stage in AGPRs) */
-template<int D0, int D1, int FMT, int NRHS, typename R>
-__device__ __forceinline__ void hop_quad(Cx<R> (&acc)[12], const vec2<R>* __restrict__ in, size_t SS, const SiteNb& nb,
-                                         uint32_t rhs, const void* gauge, uint32_t S, int P, uint32_t i,
-                                         const HopWeights<double>& w)
+/* The eight hops of the shapes with four hops' loads in flight (one wave per SIMD, which may stage in AGPRs, or
+ * two for FP32).  The four in-plane neighbours (X and Y directions) are gathered component by component: the rows
+ * of a block's sites are each other's y neighbours and every site is the x neighbour of two, so what one gather of
+ * a component brings into the 32 KiB L1 (4 KiB for 256 sites and one 16-byte component) the next ones find there.
+ * Gathering spinor by spinor (two directions at a time, four spinors of 48 KiB each per block) found none of it:
+ * the L1 asked the L2 for every gathered byte, 112 M lines per launch at 48^3x96 in FP64.  Measured, spinor by
+ * spinor / component by component, one run: F64_18 1516 / 1481 us at 48^3x96, 98.9 / 94.3 us at 24^3x48, 289 /
+ * 279 us at 32^3x64; F64_12 1147 / 1143 us and F32 555 / 545 us at 48^3x96.  The hops are applied in the order
+ * T, X, Y, Z (the X and Y links are loaded once the T hops have freed their registers, the Z hops' data once the X
+ * hops have), so every variant computes the same bits. */
+template<int FMT, int NRHS, typename R>
+__device__ __forceinline__ void hop_all(Cx<R> (&acc)[12], const vec2<R>* __restrict__ in, size_t SS, const SiteNb& nb,
+                                        uint32_t rhs, const void* gauge, uint32_t S, int P, uint32_t i,
+                                        const HopWeights<double>& w)
 {
-    Su3<R> u0f, u0b, u1f, u1b;
-    vec2<R> s0f[12], s0b[12], s1f[12], s1b[12];
-    GaugeLoad<FMT>::load(gauge, S, D0, P, i, u0f);
-    GaugeLoad<FMT>::load(gauge, S, D0, P ^ 1, nb.dn[D0], u0b);
-    GaugeLoad<FMT>::load(gauge, S, D1, P, i, u1f);
-    GaugeLoad<FMT>::load(gauge, S, D1, P ^ 1, nb.dn[D1], u1b);
-    load_spinor<R>(s0f, in, SS, (size_t)nb.up[D0] * NRHS + rhs);
-    load_spinor<R>(s0b, in, SS, (size_t)nb.dn[D0] * NRHS + rhs);
-    load_spinor<R>(s1f, in, SS, (size_t)nb.up[D1] * NRHS + rhs);
-    load_spinor<R>(s1b, in, SS, (size_t)nb.dn[D1] * NRHS + rhs);
-    apply_hop<D0, true>(acc, s0f, u0f, Cx<R>{R(w.wf[D0][0]), R(w.wf[D0][1])});
-    apply_hop<D0, false>(acc, s0b, u0b, Cx<R>{R(w.wb[D0][0]), R(w.wb[D0][1])});
-    apply_hop<D1, true>(acc, s1f, u1f, Cx<R>{R(w.wf[D1][0]), R(w.wf[D1][1])});
-    apply_hop<D1, false>(acc, s1b, u1b, Cx<R>{R(w.wb[D1][0]), R(w.wb[D1][1])});
+    vec2<R> sp[4][12];  // x + X, x - X, x + Y, x - Y
+    {
+        Su3<R> uf, ub;
+        vec2<R> sf[12], sb[12];
+        GaugeLoad<FMT>::load(gauge, S, 0, P, i, uf);
+        GaugeLoad<FMT>::load(gauge, S, 0, P ^ 1, nb.dn[0], ub);
+        load_spinor<R>(sf, in, SS, (size_t)nb.up[0] * NRHS + rhs);
+        load_spinor<R>(sb, in, SS, (size_t)nb.dn[0] * NRHS + rhs);
+        const size_t o[4] = {(size_t)nb.up[1] * NRHS + rhs, (size_t)nb.dn[1] * NRHS + rhs,
+                             (size_t)nb.up[2] * NRHS + rhs, (size_t)nb.dn[2] * NRHS + rhs};
+        load_spinors_interleaved<R, 4>(sp, in, SS, o);
+        apply_hop<0, true>(acc, sf, uf, Cx<R>{R(w.wf[0][0]), R(w.wf[0][1])});
+        apply_hop<0, false>(acc, sb, ub, Cx<R>{R(w.wb[0][0]), R(w.wb[0][1])});
+    }
+    Su3<R> xf, xb, yf, yb, zf, zb;
+    vec2<R> szf[12], szb[12];
+    GaugeLoad<FMT>::load(gauge, S, 1, P, i, xf);
+    GaugeLoad<FMT>::load(gauge, S, 1, P ^ 1, nb.dn[1], xb);
+    GaugeLoad<FMT>::load(gauge, S, 2, P, i, yf);
+    GaugeLoad<FMT>::load(gauge, S, 2, P ^ 1, nb.dn[2], yb);
+    apply_hop<1, true>(acc, sp[0], xf, Cx<R>{R(w.wf[1][0]), R(w.wf[1][1])});
+    apply_hop<1, false>(acc, sp[1], xb, Cx<R>{R(w.wb[1][0]), R(w.wb[1][1])});
+    GaugeLoad<FMT>::load(gauge, S, 3, P, i, zf);
+    GaugeLoad<FMT>::load(gauge, S, 3, P ^ 1, nb.dn[3], zb);
+    load_spinor<R>(szf, in, SS, (size_t)nb.up[3] * NRHS + rhs);
+    load_spinor<R>(szb, in, SS, (size_t)nb.dn[3] * NRHS + rhs);
+    apply_hop<2, true>(acc, sp[2], yf, Cx<R>{R(w.wf[2][0]), R(w.wf[2][1])});
+    apply_hop<2, false>(acc, sp[3], yb, Cx<R>{R(w.wb[2][0]), R(w.wb[2][1])});
+    apply_hop<3, true>(acc, szf, zf, Cx<R>{R(w.wf[3][0]), R(w.wf[3][1])});
+    apply_hop<3, false>(acc, szb, zb, Cx<R>{R(w.wb[3][0]), R(w.wb[3][1])});
 }
 
 /* the same two hops one after the other, for the 128-VGPR variants: each loads only its own link and
@@ -185,8 +209,8 @@ __device__ __forceinline__ void hop_pair(Cx<R> (&acc)[12], const vec2<R>* __rest
 
 /* Register budget and hops in flight per thread:
  *   OCC = 0: at most 2 waves per SIMD (up to 256 VGPRs), the two hops of one direction in flight;
- *   OCC = 1: 1 wave per SIMD, the four hops of two directions in flight (blocks of at most 256);
- *   OCC = 2: at most 2 waves per SIMD with the four hops of two directions in flight (FP32);
+ *   OCC = 1: 1 wave per SIMD, four hops and more in flight (hop_all; blocks of at most 256);
+ *   OCC = 2: the same at at most 2 waves per SIMD (FP32);
  *   OCC = 4: at least 4 waves per SIMD (at most 128 VGPRs), one hop at a time.
  * PLAIN: the plain hopping term (no epilogue, no norms), compiled without the epilogue's branches and the
  * block reduction; same arithmetic (a standalone copy measured 0.8 % faster than the general kernel for FP64
@@ -221,8 +245,7 @@ void k_dslash_eo(DslashArgs a)
         hop_pair<m, FMT>(acc, in, SS, nb.up[m] * NRHS + rhs, nb.dn[m] * NRHS + rhs, a.gauge, S, P, i, nb.dn[m],     \
                          CL2_W(wf, m), CL2_W(wb, m));
         if constexpr (OCC == 1 || OCC == 2) {
-            hop_quad<0, 1, FMT, NRHS>(acc, in, SS, nb, rhs, a.gauge, S, P, i, a.w);
-            hop_quad<2, 3, FMT, NRHS>(acc, in, SS, nb, rhs, a.gauge, S, P, i, a.w);
+            hop_all<FMT, NRHS>(acc, in, SS, nb, rhs, a.gauge, S, P, i, a.w);
         } else {
             CL2_DIR(0)
             CL2_DIR(1)
@@ -323,7 +346,10 @@ __global__ __launch_bounds__((MrhsLds<NRHS, SBX>::BLOCK)) void k_dslash_eo_mrhs_
     // complex numbers, plus a 32-bit per-lane byte offset, which the host allows only while
     // Veo * NRHS * sizeof(V) < 2^32.  That removes the per-lane 64-bit address arithmetic and brings the
     // kernel from 3 to 4 waves per SIMD (measured 25 % faster at 12 right-hand sides); for FP32 the
-    // 64-bit form measured 1-3 % faster.
+    // 64-bit form measured 1-3 % faster.  FP32 gathers the two neighbours of a direction pair by pair, in that
+    // order (the empty asm holds it): x + X and x - X share their cache lines, which are still in the L1 then
+    // (spinor by spinor 600 us, pair by pair 577 us for 8 right-hand sides at 32^3x64; 12: 879 / 875 us at
+    // 32^3x64, 49.5 / 46.6 us at 16^3x32).
     constexpr bool NARROW = sizeof(R) == 8 && !WIDE;
     const V* in = reinterpret_cast<const V*>(a.in);
     gchar_ptr cb[12];
@@ -345,8 +371,15 @@ __global__ __launch_bounds__((MrhsLds<NRHS, SBX>::BLOCK)) void k_dslash_eo_mrhs_
         } else {                                                                                                \
             const size_t ef = (size_t)lnb[s * 8 + 2 * (m)] * NRHS + rhs;                                        \
             const size_t eb = (size_t)lnb[s * 8 + 2 * (m) + 1] * NRHS + rhs;                                    \
-            load_spinor<R>(sf, in, SS, ef);                                                                     \
-            load_spinor<R>(sb, in, SS, eb);                                                                     \
+            if constexpr (sizeof(R) == 4) {                                                                     \
+                vec2<R> sp[2][12];                                                                              \
+                const size_t o2[2] = {ef, eb};                                                                  \
+                load_spinors_interleaved<R, 2>(sp, in, SS, o2);                                                 \
+                _Pragma("unroll") for (int k = 0; k < 12; ++k) sf[k] = sp[0][k], sb[k] = sp[1][k];              \
+            } else {                                                                                            \
+                load_spinor<R>(sf, in, SS, ef);                                                                 \
+                load_spinor<R>(sb, in, SS, eb);                                                                 \
+            }                                                                                                   \
         }                                                                                                       \
         const Su3<R> uf = lu[s * 8 + 2 * (m)], ub = lu[s * 8 + 2 * (m) + 1];                                    \
         apply_hop<m, true>(acc, sf, uf, Cx<R>{R(a.w.wf[m][0]), R(a.w.wf[m][1])});                             \
