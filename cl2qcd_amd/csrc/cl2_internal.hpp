@@ -82,7 +82,9 @@ HopWeights<double> wilson_weights(const cl2_ctx* c, double kappa);
 hipError_t launch_dslash(cl2_ctx* c, const DslashArgs& a, int format);
 hipError_t launch_sitediag(cl2_ctx* c, void* out, const void* in, int prec, const double f1[2], const double f2[2],
                            double scale);
-hipError_t launch_dks(cl2_ctx* c, void* out, const void* in, const void* gauge, int format, int evenodd);
+/* with x: out = coef x - D in (the last step of MdagM_eo) */
+hipError_t launch_dks(cl2_ctx* c, void* out, const void* in, const void* gauge, int format, int evenodd,
+                      const void* x = nullptr, double coef = 0.);
 /* nrhs = 2, 4, 8, 12, 16 staggered vectors [3][Veo][nrhs]; with x: out_r = coef[r] x_r - D in_r */
 hipError_t launch_dks_step(cl2_ctx* c, void* out, const void* in, const void* gauge, int format, int evenodd,
                            const void* own, const void* x, double coef, void* cg_r, const double* beta,

@@ -16,8 +16,8 @@ struct DksArgs {
     int out_parity;
     double sf[4][2];  // 0.5 * b_mu (* imaginary chemical potential on T)
     WorkMap map;
-    // multi-RHS launches ([3][Veo][nrhs] fields): with x set, out_r = coef[r] x_r - D in_r (the last step of
-    // MdagM_eo with a shift per right-hand side)
+    // with x set, out_r = coef[r] x_r - D in_r (the last step of MdagM_eo; multi-RHS launches, on [3][Veo][nrhs]
+    // fields, have a shift per right-hand side)
     const void* x;
     double coef[16];
     // the fused CG step of the lockstep solver (multi-RHS only): norm_partials[r * gridDim.x + block] gets per
@@ -127,6 +127,16 @@ void k_dks_eo(DksArgs a)
                 for (int c = 0; c < 3; ++c) vb[c] = in[(size_t)c * S + nb.dn[mu]];
                 dks_hops(acc, uf, vf, ub, vb, wt(mu));
             }
+        }
+    }
+    if (a.x) {  // the MdagM_eo epilogue as the elementwise kernel computes it: coef x - out
+        const V* xv      = reinterpret_cast<const V*>(a.x);
+        const Cx<R> cf   = Cx<R>{R(a.coef[0]), R(0)};
+        const Cx<R> mone = Cx<R>{R(-1), R(0)};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const V v = xv[(size_t)c * S + i];
+            acc[c]    = cmul(Cx<R>{v.x, v.y}, cf) + cmul(acc[c], mone);
         }
     }
     V* out = reinterpret_cast<V*>(a.out);
@@ -431,7 +441,8 @@ hipError_t launch_dks_step(cl2_ctx* c, void* out, const void* in, const void* ga
     return hipGetLastError();
 }
 
-hipError_t launch_dks(cl2_ctx* c, void* out, const void* in, const void* gauge, int format, int evenodd)
+hipError_t launch_dks(cl2_ctx* c, void* out, const void* in, const void* gauge, int format, int evenodd, const void* x,
+                      double coef)
 {
     DksArgs a;
     a.in         = in;
@@ -439,7 +450,8 @@ hipError_t launch_dks(cl2_ctx* c, void* out, const void* in, const void* gauge, 
     a.gauge      = gauge;
     a.g          = c->g;
     a.out_parity = evenodd;
-    a.x          = nullptr;
+    a.x          = x;
+    a.coef[0]    = coef;
     const cl2_hop_tuning t = hop_tuning(c, format | DKS_TUNING_KEY, 1);
     const int bs           = (t.block == 128 || t.block == 512) ? t.block : 256;
     a.map                  = work_map(c, bs, 1, t);
