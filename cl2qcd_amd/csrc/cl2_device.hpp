@@ -239,6 +239,13 @@ __device__ __forceinline__ vec2<R> load_at(gchar_ptr base, uint32_t off)
     return vec2<R>{v.x, v.y};
 }
 
+__device__ __forceinline__ float4 load4_at(gchar_ptr base, uint32_t off)
+{
+    typedef float N __attribute__((ext_vector_type(4)));
+    const N v = *(const __attribute__((address_space(1))) N*)(base + off);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
 /* eo index of logical site l of the work order (l < veo) */
 __device__ __forceinline__ uint32_t logical_site(const WorkMap& m, uint32_t l)
 {

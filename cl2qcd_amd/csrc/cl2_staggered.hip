@@ -277,6 +277,159 @@ __global__ __launch_bounds__(DksMrhs<NRHS>::BLOCK) void k_dks_eo_mrhs(DksArgs a)
     }
 }
 
+/* The same for FP32 with two adjacent right-hand sides per thread: their 8-byte elements are one 16-byte lane, so
+ * gathers, epilogue loads and stores take half the instructions per byte, and each link read from LDS, neighbour
+ * index and address serves two right-hand sides.  The one-per-thread kernel was bound by instruction issue (703
+ * vector instructions per wave for 288 of link arithmetic).  Gather offsets are 32-bit from a scalar base per
+ * component.  Taken for 8, 12 and 16 right-hand sides (for 2 and 4 a block is one or two waves and the chip is left
+ * with fewer of them: no gain at 24^3x24, 6.6 against 5.7 us at 12^4), 16-byte aligned fields and Veo nrhs 8 bytes
+ * < 4 GiB; k_dks_eo_mrhs takes the rest.  Per right-hand side the arithmetic is unchanged (same bits); the norm
+ * partials cover 32 sites, half as many as before for stage 2 to sum.  One D_KS_eo, one / two right-hand sides per
+ * thread: 240 / 205 us for 16 at 48^3x12, 46.1 / 40.6 us for 12 and 35.1 / 31.5 us for 8 at 24^4. */
+template<int NRHS>
+struct DksPair {
+    static constexpr int T     = NRHS / 2;                              // threads per site
+    static constexpr int SB    = 32;                                    // sites per block
+    static constexpr int BLOCK = SB * T;
+};
+
+template<int NRHS>
+__global__ __launch_bounds__(DksPair<NRHS>::BLOCK) void k_dks_eo_mrhs_pair(DksArgs a)
+{
+    constexpr int T     = DksPair<NRHS>::T;
+    constexpr int SB    = DksPair<NRHS>::SB;
+    constexpr int BLOCK = DksPair<NRHS>::BLOCK;
+    __shared__ Su3<float> lu[SB * 8];
+    __shared__ uint32_t lnb[SB * 8];
+    __shared__ uint32_t lsite[SB];
+    __shared__ double2 lred[BLOCK * 2];
+    const uint32_t S  = a.g.veo;
+    const size_t SS   = (size_t)S * NRHS;
+    const uint32_t Lb = logical_block(a.map, blockIdx.x);
+    const int P       = a.out_parity;
+    if (threadIdx.x < SB) {
+        const uint32_t l = Lb * SB + threadIdx.x;
+        const uint32_t i = logical_site(a.map, l < S ? l : S - 1);
+        SiteNb nb;
+        site_neighbours(a.g, i, P, nb);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            lnb[threadIdx.x * 8 + 2 * d]     = nb.up[d];
+            lnb[threadIdx.x * 8 + 2 * d + 1] = nb.dn[d];
+        }
+        lsite[threadIdx.x] = i;
+    }
+    __syncthreads();
+    for (int w = threadIdx.x; w < SB * 8; w += BLOCK) {
+        const int h = w & 7;
+        Su3<float> u;
+        GaugeLoad<GAUGE_F32_12>::load(a.gauge, S, h >> 1, (h & 1) ? P ^ 1 : P, (h & 1) ? lnb[w] : lsite[w >> 3], u);
+        lu[w] = u;
+    }
+    __syncthreads();
+    const int s      = threadIdx.x / T;
+    const int pr     = threadIdx.x - s * T;
+    const uint32_t i = lsite[s];
+    double2 sum[2]   = {make_double2(0., 0.), make_double2(0., 0.)};
+    if (Lb * SB + s < S) {
+        uint32_t x, y, z, t;
+        site_coords(a.g, i, P, x, y, z, t);
+        const float eta[4] = {((x + y + z) & 1u) ? -1.f : 1.f, 1.f, (x & 1u) ? -1.f : 1.f, ((x + y) & 1u) ? -1.f : 1.f};
+        gchar_ptr cb[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            cb[c] = uniform_ptr(reinterpret_cast<const char*>(a.in) + (size_t)c * SS * sizeof(float2));
+        Cx<float> acc[2][3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) acc[0][k] = acc[1][k] = Cx<float>{0.f, 0.f};
+#pragma unroll
+        for (int mu = 0; mu < 4; ++mu) {
+            float4 vf[3], vb[3];
+            const uint32_t ef = (lnb[s * 8 + 2 * mu] * T + pr) * (uint32_t)sizeof(float4);
+            const uint32_t eb = (lnb[s * 8 + 2 * mu + 1] * T + pr) * (uint32_t)sizeof(float4);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) vf[c] = load4_at(cb[c], ef);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) vb[c] = load4_at(cb[c], eb);
+            const Su3<float> uf = lu[s * 8 + 2 * mu], ub = lu[s * 8 + 2 * mu + 1];
+            const Cx<float> w{(float)a.sf[mu][0] * eta[mu], (float)a.sf[mu][1] * eta[mu]};
+            const float2 f0[3] = {{vf[0].x, vf[0].y}, {vf[1].x, vf[1].y}, {vf[2].x, vf[2].y}};
+            const float2 f1[3] = {{vf[0].z, vf[0].w}, {vf[1].z, vf[1].w}, {vf[2].z, vf[2].w}};
+            const float2 b0[3] = {{vb[0].x, vb[0].y}, {vb[1].x, vb[1].y}, {vb[2].x, vb[2].y}};
+            const float2 b1[3] = {{vb[0].z, vb[0].w}, {vb[1].z, vb[1].w}, {vb[2].z, vb[2].w}};
+            dks_hops(acc[0], uf, f0, ub, b0, w);
+            dks_hops(acc[1], uf, f1, ub, b1, w);
+        }
+        const size_t o  = (size_t)i * T + pr;
+        const size_t S4 = SS / 2;
+        if (a.x) {  // the MdagM_eo epilogue as the elementwise kernel computes it: coef x - out
+            const float4* xv     = reinterpret_cast<const float4*>(a.x);
+            const Cx<float> c0{(float)a.coef[2 * pr], 0.f}, c1{(float)a.coef[2 * pr + 1], 0.f};
+            const Cx<float> mone{-1.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const float4 v = xv[(size_t)c * S4 + o];
+                acc[0][c]      = cmul(Cx<float>{v.x, v.y}, c0) + cmul(acc[0][c], mone);
+                acc[1][c]      = cmul(Cx<float>{v.z, v.w}, c1) + cmul(acc[1][c], mone);
+            }
+        }
+        auto add2 = [](double& d, float p, float q) { d += (double)p * (double)p + (double)q * (double)q; };
+        if (a.cg_r) {  // r <- r - alpha A p, A p never stored
+            float4* rp = reinterpret_cast<float4*>(a.cg_r);
+            const Cx<float> a0{(float)a.cg_alpha[4 * pr], (float)a.cg_alpha[4 * pr + 1]};
+            const Cx<float> a1{(float)a.cg_alpha[4 * pr + 2], (float)a.cg_alpha[4 * pr + 3]};
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const float4 ro    = rp[(size_t)c * S4 + o];
+                const Cx<float> r0 = Cx<float>{ro.x, ro.y} - cmul(acc[0][c], a0);
+                const Cx<float> r1 = Cx<float>{ro.z, ro.w} - cmul(acc[1][c], a1);
+                store_stream(rp + (size_t)c * S4 + o, make_float4(r0.re, r0.im, r1.re, r1.im));
+                add2(sum[0].x, r0.re, r0.im);
+                add2(sum[1].x, r1.re, r1.im);
+                sum[0].y += (double)r0.re * (double)ro.x + (double)r0.im * (double)ro.y;
+                sum[1].y += (double)r1.re * (double)ro.z + (double)r1.im * (double)ro.w;
+            }
+        } else {
+            float4* out = reinterpret_cast<float4*>(a.out);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                store_stream(out + (size_t)c * S4 + o,
+                             make_float4(acc[0][c].re, acc[0][c].im, acc[1][c].re, acc[1][c].im));
+            if (a.norm_partials) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    add2(sum[0].x, acc[0][c].re, acc[0][c].im);
+                    add2(sum[1].x, acc[1][c].re, acc[1][c].im);
+                }
+                if (a.own) {
+                    const float4* ov = reinterpret_cast<const float4*>(a.own);
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const float4 v = ov[(size_t)c * S4 + o];
+                        add2(sum[0].y, v.x, v.y);
+                        add2(sum[1].y, v.z, v.w);
+                    }
+                }
+            }
+        }
+    }
+    if (a.norm_partials) {
+        // per right-hand side: thread r < NRHS sums the SB site threads of its column in site order
+        lred[threadIdx.x * 2]     = sum[0];
+        lred[threadIdx.x * 2 + 1] = sum[1];
+        __syncthreads();
+        if ((int)threadIdx.x < NRHS) {
+            double2 tsum = make_double2(0., 0.);
+#pragma unroll 8
+            for (int q = 0; q < SB; ++q) {
+                tsum.x += lred[q * NRHS + threadIdx.x].x;
+                tsum.y += lred[q * NRHS + threadIdx.x].y;
+            }
+            a.norm_partials[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = tsum;
+        }
+    }
+}
+
 static void dks_weights(cl2_ctx* c, DksArgs& a)
 {
     for (int mu = 0; mu < 4; ++mu) {
@@ -311,8 +464,22 @@ hipError_t launch_dks_mrhs(cl2_ctx* c, void* out, const void* in, const void* ga
     for (int r = 0; r < 16; ++r) a.coef[r] = (x && r < nrhs) ? coef[r] : 0.;
     dks_weights(c, a);
     const cl2_hop_tuning t = hop_tuning(c, format | DKS_TUNING_KEY, 1);
+    const bool pairs = format == GAUGE_F32_12 && mrhs_offsets_narrow(c->g.veo, nrhs, sizeof(float2)) &&
+                       ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(in) |
+                         reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(own) |
+                         reinterpret_cast<uintptr_t>(cg_r)) & 15u) == 0;
     auto go = [&](auto fmt_tag, auto n_tag) -> hipError_t {
         constexpr int F = decltype(fmt_tag)::value, N = decltype(n_tag)::value;
+        if constexpr (F == GAUGE_F32_12 && N >= 8) {
+            if (pairs) {
+                constexpr int SB = DksPair<N>::SB;
+                const unsigned nb = (c->g.veo + SB - 1) / SB;
+                a.map             = work_map(c, SB, 1, t);
+                if (nblocks) *nblocks = nb;
+                hipLaunchKernelGGL((k_dks_eo_mrhs_pair<N>), dim3(nb), dim3(DksPair<N>::BLOCK), 0, c->stream, a);
+                return hipGetLastError();
+            }
+        }
         constexpr int SB = DksMrhs<N>::SB;
         a.map = work_map(c, SB, 1, t);
         if (nblocks) *nblocks = (c->g.veo + SB - 1) / SB;
