@@ -249,18 +249,14 @@ hipError_t launch_reduce_stage1(cl2_ctx* c, const void* x, const void* y, size_t
 /* stage 2: one block sums the partials in a fixed order.
  * out_kind 0: res[0] = re;  1: res = (re, im);  2: res[k] = alpha[k]^2 * re for k < nvec;
  * 3: res = (re, im, re, 0) */
-template<int BLOCK>
+template<int BLOCK, bool WIDE>
 __global__ __launch_bounds__(BLOCK) void k_reduce2(const double* __restrict__ partials, unsigned nparts,
                                                    double* __restrict__ res, int out_kind,
                                                    const double* __restrict__ alpha, int nvec)
 {
     __shared__ double lds[2 * BLOCK / 64];
-    double2 acc = make_double2(0., 0.);
-    for (unsigned k = threadIdx.x; k < nparts; k += BLOCK) {
-        acc.x += partials[2 * k];
-        acc.y += partials[2 * k + 1];
-    }
-    double2 s = block_sum2<BLOCK>(acc, lds);
+    const double2 s =
+        block_sum2<BLOCK>(strided_sum<BLOCK, WIDE>(reinterpret_cast<const double2*>(partials), nparts), lds);
     if (threadIdx.x == 0) {
         if (out_kind == 0) {
             res[0] = s.x;
@@ -282,8 +278,13 @@ hipError_t launch_reduce_stage2(cl2_ctx* c, unsigned nparts, double* res, int ou
                                 int nvec, const double* parts)
 {
     // 1024 threads: the elementwise kernels leave up to BLAS_MAX_BLOCKS partials
-    hipLaunchKernelGGL((k_reduce2<1024>), dim3(1), dim3(1024), 0, c->stream, parts ? parts : c->partials, nparts, res,
-                       out_kind, alpha_vec, nvec);
+    const double* p = parts ? parts : c->partials;
+    if (nparts >= WIDE_SUM_MIN(1024))
+        hipLaunchKernelGGL((k_reduce2<1024, true>), dim3(1), dim3(1024), 0, c->stream, p, nparts, res, out_kind,
+                           alpha_vec, nvec);
+    else
+        hipLaunchKernelGGL((k_reduce2<1024, false>), dim3(1), dim3(1024), 0, c->stream, p, nparts, res, out_kind,
+                           alpha_vec, nvec);
     return hipGetLastError();
 }
 

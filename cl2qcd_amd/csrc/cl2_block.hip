@@ -228,18 +228,12 @@ __global__ __launch_bounds__(256) void k_block_dot(const void* x, const void* y,
 
 /* stage 2: block r sums right-hand side r's nb partials; out_kind 0: res[2r..2r+1] = complex sum,
  * 1: res[r] = real part */
-template<int BLOCK>
+template<int BLOCK, bool WIDE>
 __global__ __launch_bounds__(BLOCK) void k_block_reduce2(const double2* partials, unsigned nb, double* res,
                                                          int out_kind)
 {
     __shared__ double lds[2 * BLOCK / 64];
-    const double2* p = partials + (size_t)blockIdx.x * nb;
-    double2 acc      = make_double2(0., 0.);
-    for (unsigned k = threadIdx.x; k < nb; k += BLOCK) {
-        acc.x += p[k].x;
-        acc.y += p[k].y;
-    }
-    const double2 s = block_sum2<BLOCK>(acc, lds);
+    const double2 s = block_sum2<BLOCK>(strided_sum<BLOCK, WIDE>(partials + (size_t)blockIdx.x * nb, nb), lds);
     if (threadIdx.x == 0) {
         if (out_kind == 0) {
             res[2 * blockIdx.x]     = s.x;
@@ -396,7 +390,12 @@ constexpr int BLOCK_U_REDUCE = 4;
 
 hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, double* res, int out_kind, int nrhs)
 {
-    hipLaunchKernelGGL((k_block_reduce2<1024>), dim3(nrhs), dim3(1024), 0, c->stream, parts, nb, res, out_kind);
+    if (nb >= WIDE_SUM_MIN(1024))
+        hipLaunchKernelGGL((k_block_reduce2<1024, true>), dim3(nrhs), dim3(1024), 0, c->stream, parts, nb, res,
+                           out_kind);
+    else
+        hipLaunchKernelGGL((k_block_reduce2<1024, false>), dim3(nrhs), dim3(1024), 0, c->stream, parts, nb, res,
+                           out_kind);
     return hipGetLastError();
 }
 
