@@ -103,6 +103,24 @@ __device__ __forceinline__ Cx<R> add_unit(Cx<R> a, Cx<R> b)
     return Cx<R>{a.re + b.im, a.im - b.re};
 }
 
+/* The projector (1 - gamma_mu) (forward) or (1 + gamma_mu) (backward) as rows h = s_A + C s_B for A = row = 0, 1:
+ * the spin B and the unit C of a row, and the conjugate of a unit. */
+__host__ __device__ constexpr int hop_b(int dir, int row)
+{
+    return (dir == 0 || dir == 3) ? 2 + row : 3 - row;
+}
+__host__ __device__ constexpr int hop_unit(int dir, bool fwd, int row)
+{
+    const bool plus = dir < 2 ? fwd : (fwd == (row == 0));
+    return (dir == 0 || dir == 2) ? (plus ? P1 : M1) : (plus ? PI : MI);
+}
+__host__ __device__ constexpr int unit_conj(int u)
+{
+    return u == PI ? MI : (u == MI ? PI : u);
+}
+/* block shape of the wave-per-hop kernels: 64 sites, one wave for each of the eight hops */
+constexpr int SPLIT_SITES = 64, SPLIT_BLOCK = 8 * SPLIT_SITES;
+
 template<typename R>
 struct Su3 {
     Cx<R> e[3][3];

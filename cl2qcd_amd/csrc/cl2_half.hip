@@ -347,6 +347,188 @@ void k_dslash_eo_h(DslashArgs a)
     }
 }
 
+/* acc += U w r for one component: U = 1 for the upper row of a projector, conj(C) for the lower; RW: real weight
+ * (the two forms of half_hop_r) */
+template<int U, bool RW>
+__device__ __forceinline__ void add_weighted(Cx<float>& y, Cx<float> r, Cx<float> w)
+{
+    if constexpr (RW) {
+        const float wr = w.re;
+        if constexpr (U == P1) y = Cx<float>{__builtin_fmaf(r.re, wr, y.re), __builtin_fmaf(r.im, wr, y.im)};
+        if constexpr (U == M1) y = Cx<float>{__builtin_fmaf(r.re, -wr, y.re), __builtin_fmaf(r.im, -wr, y.im)};
+        if constexpr (U == PI) y = Cx<float>{__builtin_fmaf(r.im, -wr, y.re), __builtin_fmaf(r.re, wr, y.im)};
+        if constexpr (U == MI) y = Cx<float>{__builtin_fmaf(r.im, wr, y.re), __builtin_fmaf(r.re, -wr, y.im)};
+    } else {
+        y = add_unit<U>(y, cmul(r, w));
+    }
+}
+
+/* the rows of one hop, r_A = (U or U^dagger) (s_A + C s_B) for A = 0, 1 (half_hop_r without the weight) */
+template<int DIR, bool FWD>
+__device__ __forceinline__ void hop_rows_h(Cx<float> (&r)[6], const h2 (&psi)[12], const Su3h& u)
+{
+    auto row = [&](auto row_tag) {
+        constexpr int A = decltype(row_tag)::value, B = hop_b(DIR, A), C = hop_unit(DIR, FWD, A);
+        h2 f1[3], f2[3];
+        Cx<float> v[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) proj_h<C, FWD>(psi[3 * A + c], psi[3 * B + c], f1[c], f2[c]);
+        su3_dot_h<FWD, false>(u, f1, f2, v);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) r[3 * A + c] = v[c];
+    };
+    row(std::integral_constant<int, 0>{});
+    row(std::integral_constant<int, 1>{});
+}
+
+/* components 2Q and 2Q + 1 of the hop sum of one site, from the rows and weights of its eight hops in LDS */
+template<int Q, bool RS>
+__device__ __forceinline__ void pair_sum_h(Cx<float> (&acc)[2], const float2* rows, const float2* weights, int lane)
+{
+    auto add = [&](auto j_tag, auto h_tag) {
+        constexpr int k = 2 * Q + decltype(j_tag)::value, h = decltype(h_tag)::value;
+        constexpr int sp = k / 3, c = k % 3, dir = h >> 1;
+        constexpr int row = sp < 2 ? sp : (hop_b(dir, 0) == sp ? 0 : 1);
+        constexpr int u   = sp < 2 ? (int)P1 : unit_conj(hop_unit(dir, (h & 1) == 0, row));
+        const float2 v = rows[(h * 6 + row * 3 + c) * SPLIT_SITES + lane], w = weights[h * SPLIT_SITES + lane];
+        add_weighted<u, RS && dir != 0>(acc[decltype(j_tag)::value], Cx<float>{v.x, v.y}, Cx<float>{w.x, w.y});
+    };
+    auto all = [&](auto j_tag) {
+        add(j_tag, std::integral_constant<int, 0>{});
+        add(j_tag, std::integral_constant<int, 1>{});
+        add(j_tag, std::integral_constant<int, 2>{});
+        add(j_tag, std::integral_constant<int, 3>{});
+        add(j_tag, std::integral_constant<int, 4>{});
+        add(j_tag, std::integral_constant<int, 5>{});
+        add(j_tag, std::integral_constant<int, 6>{});
+        add(j_tag, std::integral_constant<int, 7>{});
+    };
+    acc[0] = acc[1] = Cx<float>{0.f, 0.f};
+    all(std::integral_constant<int, 0>{});
+    all(std::integral_constant<int, 1>{});
+}
+
+/* components 2q and 2q + 1 of site i: half of a 16-byte lane, times the site's norm */
+__device__ __forceinline__ void load_pair_h(Cx<float> (&v)[2], const void* p, uint32_t S, int q, uint32_t i)
+{
+    const float n = half_norms(p, S)[i];
+    const h4 h    = reinterpret_cast<const h4*>(p)[((size_t)(q >> 1) * S + i) * 2 + (q & 1)];
+    v[0]          = Cx<float>{(float)h[0] * n, (float)h[1] * n};
+    v[1]          = Cx<float>{(float)h[2] * n, (float)h[3] * n};
+}
+
+/* The wave-per-hop kernel of small lattices on FP16 spinors (see k_dslash_eo_split): same work split, the bits of
+ * k_dslash_eo_h.  A site's new norm, the largest of its 24 numbers, comes from the six waves' maxima through LDS. */
+template<bool RS>
+__global__ __launch_bounds__(SPLIT_BLOCK) void k_dslash_eo_split_h(DslashArgs a)
+{
+    __shared__ float2 rows[8 * 6 * SPLIT_SITES];
+    __shared__ float2 weights[8 * SPLIT_SITES];
+    __shared__ float maxima[6 * SPLIT_SITES];
+    __shared__ double lds[2 * SPLIT_BLOCK / 64];
+    const uint32_t S = a.g.veo;
+    const int lane   = threadIdx.x & 63;
+    const int wave   = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    uint32_t i       = 0;
+    const bool live  = map_site<SPLIT_SITES>(a.map, S, blockIdx.x, (uint32_t)lane, i);
+    if (live) {
+        SiteNb nb;
+        site_neighbours(a.g, i, a.out_parity, nb);
+        const int P = a.out_parity;
+        Cx<float> r[6], w;
+        auto hop = [&](auto dir_tag, auto fwd_tag) {
+            constexpr int D  = decltype(dir_tag)::value;
+            constexpr bool F = decltype(fwd_tag)::value;
+            const uint32_t n = F ? nb.up[D] : nb.dn[D];
+            Su3h u;
+            h2 psi[12];
+            load_link_h(a.gauge, S, D, F ? P : P ^ 1, F ? i : n, u);
+            const float norm = load_site_h_raw(a.in, S, n, psi);
+            hop_rows_h<D, F>(r, psi, u);
+            w = F ? weight_n(a.w.wf[D], norm) : weight_n(a.w.wb[D], norm);
+        };
+        switch (wave) {
+            case 0: hop(std::integral_constant<int, 0>{}, std::true_type{}); break;
+            case 1: hop(std::integral_constant<int, 0>{}, std::false_type{}); break;
+            case 2: hop(std::integral_constant<int, 1>{}, std::true_type{}); break;
+            case 3: hop(std::integral_constant<int, 1>{}, std::false_type{}); break;
+            case 4: hop(std::integral_constant<int, 2>{}, std::true_type{}); break;
+            case 5: hop(std::integral_constant<int, 2>{}, std::false_type{}); break;
+            case 6: hop(std::integral_constant<int, 3>{}, std::true_type{}); break;
+            default: hop(std::integral_constant<int, 3>{}, std::false_type{}); break;
+        }
+#pragma unroll
+        for (int k = 0; k < 6; ++k) rows[(wave * 6 + k) * SPLIT_SITES + lane] = make_float2(r[k].re, r[k].im);
+        weights[wave * SPLIT_SITES + lane] = make_float2(w.re, w.im);
+    }
+    __syncthreads();
+    const bool sums = live && wave < 6;
+    double nrm = 0., ry = 0.;
+    Cx<float> acc[2];
+    if (sums) {
+        switch (wave) {
+            case 0: pair_sum_h<0, RS>(acc, rows, weights, lane); break;
+            case 1: pair_sum_h<1, RS>(acc, rows, weights, lane); break;
+            case 2: pair_sum_h<2, RS>(acc, rows, weights, lane); break;
+            case 3: pair_sum_h<3, RS>(acc, rows, weights, lane); break;
+            case 4: pair_sum_h<4, RS>(acc, rows, weights, lane); break;
+            default: pair_sum_h<5, RS>(acc, rows, weights, lane); break;
+        }
+        const bool upper  = wave < 3;  // spins 0 and 1
+        const Cx<float> f = upper ? Cx<float>{float(a.f1[0]), float(a.f1[1])} : Cx<float>{float(a.f2[0]), float(a.f2[1])};
+        if (a.epilogue == EPI_MINV) {
+            const float s = float(a.scale);
+            acc[0]        = scale(cmul(acc[0], f), s);
+            acc[1]        = scale(cmul(acc[1], f), s);
+        } else if (a.epilogue == EPI_AEE) {
+            Cx<float> x[2];
+            load_pair_h(x, a.x, S, wave, i);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[j] = cmul(x[j], f) - acc[j];
+                if (a.gamma5 && !upper) acc[j] = Cx<float>{-acc[j].re, -acc[j].im};
+            }
+        }
+        if (a.cg_r) {  // the CG residual in place of the result
+            const Cx<float> al{float(a.cg_alpha[0]), float(a.cg_alpha[1])};
+            Cx<float> ro[2];
+            load_pair_h(ro, a.cg_r, S, wave, i);
+            float t = 0.f;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[j] = ro[j] - cmul(acc[j], al);
+                t      = __builtin_fmaf(acc[j].im, ro[j].im, __builtin_fmaf(acc[j].re, ro[j].re, t));
+            }
+            ry = (double)t;
+        }
+        if (a.norm_partials) {
+            float t = 0.f;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                t = __builtin_fmaf(acc[j].im, acc[j].im, __builtin_fmaf(acc[j].re, acc[j].re, t));
+            nrm = (double)t;
+        }
+        maxima[wave * SPLIT_SITES + lane] = fmaxf(fmaxf(fabsf(acc[0].re), fabsf(acc[0].im)),
+                                                  fmaxf(fabsf(acc[1].re), fabsf(acc[1].im)));
+    }
+    __syncthreads();  // also: every wave has read the old norm of the residual before wave 0 writes the new one
+    if (sums) {
+        float m = 0.f;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) m = fmaxf(m, maxima[q * SPLIT_SITES + lane]);
+        const float inv = m > 0.f ? 1.f / m : 0.f;
+        void* out       = a.cg_r ? a.cg_r : a.out;
+        const h4 h      = {(_Float16)(acc[0].re * inv), (_Float16)(acc[0].im * inv), (_Float16)(acc[1].re * inv),
+                           (_Float16)(acc[1].im * inv)};
+        reinterpret_cast<h4*>(out)[((size_t)(wave >> 1) * S + i) * 2 + (wave & 1)] = h;
+        if (wave == 0) half_norms(out, S)[i] = m;
+    }
+    if (a.norm_partials) {
+        const double2 s = block_sum2<SPLIT_BLOCK>(make_double2(nrm, ry), lds);
+        if (threadIdx.x == 0) a.norm_partials[2 * blockIdx.x] = s.x, a.norm_partials[2 * blockIdx.x + 1] = s.y;
+    }
+}
+
 /* whether the X, Y, Z hop weights have no imaginary part (no spatial boundary phase): the kernels then
  * multiply by them as reals */
 static bool spatial_weights_real(const HopWeights<double>& w)
@@ -360,9 +542,17 @@ static bool spatial_weights_real(const HopWeights<double>& w)
  * hop at a time, 0: two, 1: four) */
 hipError_t launch_dslash_h(cl2_ctx* c, const DslashArgs& a)
 {
+    const bool rs = spatial_weights_real(a.w);
+    if (a.block == SPLIT_SITES) {
+        const unsigned ns = blocks_for(a.g.veo, SPLIT_SITES);
+        if (rs)
+            hipLaunchKernelGGL(k_dslash_eo_split_h<true>, dim3(ns), dim3(SPLIT_BLOCK), 0, c->stream, a);
+        else
+            hipLaunchKernelGGL(k_dslash_eo_split_h<false>, dim3(ns), dim3(SPLIT_BLOCK), 0, c->stream, a);
+        return hipGetLastError();
+    }
     const int bs      = (a.block == 128 || a.block == 512) ? a.block : 256;
     const unsigned nb = blocks_for(a.g.veo, bs);
-    const bool rs = spatial_weights_real(a.w);
     auto go = [&](auto block_tag) {
         constexpr int B = decltype(block_tag)::value;
         auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(nb), dim3(B), 0, c->stream, a); };

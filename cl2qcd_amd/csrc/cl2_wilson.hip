@@ -271,6 +271,177 @@ void k_dslash_eo(DslashArgs a)
     }
 }
 
+/* ---- the hopping kernel of small lattices: a wave per hop ----
+ * A lattice of a few thousand eo sites fills few compute units with one thread per site, and each of its threads then
+ * works through eight hops one after the other (8.9 us for an 8^4 lattice, 8 blocks).  Here a block of eight waves
+ * owns 64 consecutive sites of the work order and wave h computes hop h of all of them (h = 2 dir + backward: every
+ * wave runs one straight piece of code, and its link and spinor loads stay contiguous); the hops' half spinors meet
+ * in LDS, where waves 0..5 add up two components each in the order T, X, Y, Z, forward then backward, and apply the
+ * epilogue.  The arithmetic and its order are those of k_dslash_eo: same bits (the norm partials group the
+ * components differently).  Figures and the sizes it is taken for: wave_per_hop. */
+/* w (U or U^dagger) (s_A + C s_B) for both rows of one hop */
+template<int DIR, bool FWD, typename R>
+__device__ __forceinline__ void hop_rows(Cx<R> (&t)[6], const vec2<R> (&s)[12], const Su3<R>& u, Cx<R> w)
+{
+    auto row = [&](auto row_tag) {
+        constexpr int A = decltype(row_tag)::value, B = hop_b(DIR, A), C = hop_unit(DIR, FWD, A);
+        Cx<R> h[3], r[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            h[c] = add_unit<C>(Cx<R>{s[3 * A + c].x, s[3 * A + c].y}, Cx<R>{s[3 * B + c].x, s[3 * B + c].y});
+        if constexpr (FWD)
+            su3_times(u, h, r);
+        else
+            su3dag_times(u, h, r);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) t[3 * A + c] = cmul(r[c], w);
+    };
+    row(std::integral_constant<int, 0>{});
+    row(std::integral_constant<int, 1>{});
+}
+
+/* components 2Q and 2Q + 1 of the hop sum of one site, from the rows of its eight hops in LDS */
+template<int Q, typename R>
+__device__ __forceinline__ void pair_sum(Cx<R> (&acc)[2], const vec2<R>* rows, int lane)
+{
+    auto add = [&](auto j_tag, auto h_tag) {
+        constexpr int k = 2 * Q + decltype(j_tag)::value, h = decltype(h_tag)::value;
+        constexpr int sp = k / 3, c = k % 3, dir = h >> 1;
+        constexpr int row = sp < 2 ? sp : (hop_b(dir, 0) == sp ? 0 : 1);
+        constexpr int u   = sp < 2 ? (int)P1 : unit_conj(hop_unit(dir, (h & 1) == 0, row));
+        const vec2<R> v   = rows[(h * 6 + row * 3 + c) * SPLIT_SITES + lane];
+        Cx<R>& a          = acc[decltype(j_tag)::value];
+        a                 = add_unit<u>(a, Cx<R>{v.x, v.y});
+    };
+    auto all = [&](auto j_tag) {
+        add(j_tag, std::integral_constant<int, 0>{});
+        add(j_tag, std::integral_constant<int, 1>{});
+        add(j_tag, std::integral_constant<int, 2>{});
+        add(j_tag, std::integral_constant<int, 3>{});
+        add(j_tag, std::integral_constant<int, 4>{});
+        add(j_tag, std::integral_constant<int, 5>{});
+        add(j_tag, std::integral_constant<int, 6>{});
+        add(j_tag, std::integral_constant<int, 7>{});
+    };
+    acc[0] = acc[1] = Cx<R>{R(0), R(0)};
+    all(std::integral_constant<int, 0>{});
+    all(std::integral_constant<int, 1>{});
+}
+
+/* components 2q and 2q + 1 of site i of a spinor field of S sites */
+template<typename R>
+__device__ __forceinline__ void load_pair(vec2<R> (&v)[2], const void* p, size_t S, int q, size_t i)
+{
+    if constexpr (sizeof(R) == 8) {
+        v[0] = reinterpret_cast<const vec2<R>*>(p)[(size_t)(2 * q) * S + i];
+        v[1] = reinterpret_cast<const vec2<R>*>(p)[(size_t)(2 * q + 1) * S + i];
+    } else {
+        const float4 w = reinterpret_cast<const float4*>(p)[(size_t)q * S + i];
+        v[0]           = vec2<R>{w.x, w.y};
+        v[1]           = vec2<R>{w.z, w.w};
+    }
+}
+template<typename R>
+__device__ __forceinline__ void store_pair(void* p, size_t S, int q, size_t i, Cx<R> a, Cx<R> b)
+{
+    if constexpr (sizeof(R) == 8) {
+        reinterpret_cast<vec2<R>*>(p)[(size_t)(2 * q) * S + i]     = vec2<R>{a.re, a.im};
+        reinterpret_cast<vec2<R>*>(p)[(size_t)(2 * q + 1) * S + i] = vec2<R>{b.re, b.im};
+    } else {
+        reinterpret_cast<float4*>(p)[(size_t)q * S + i] = make_float4(a.re, a.im, b.re, b.im);
+    }
+}
+
+template<int FMT>
+__global__ __launch_bounds__(SPLIT_BLOCK) void k_dslash_eo_split(DslashArgs a)
+{
+    using R = typename GaugeLoad<FMT>::R;
+    using V = vec2<R>;
+    __shared__ V rows[8 * 6 * SPLIT_SITES];
+    __shared__ double lds[2 * SPLIT_BLOCK / 64];
+    const uint32_t S = a.g.veo;
+    const int lane   = threadIdx.x & 63;
+    const int wave   = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    uint32_t i       = 0;
+    const bool live  = map_site<SPLIT_SITES>(a.map, S, blockIdx.x, (uint32_t)lane, i);
+    if (live) {
+        SiteNb nb;
+        site_neighbours(a.g, i, a.out_parity, nb);
+        const V* in = reinterpret_cast<const V*>(a.in);
+        const int P = a.out_parity;
+        Cx<R> t[6];
+        auto hop = [&](auto dir_tag, auto fwd_tag) {
+            constexpr int D  = decltype(dir_tag)::value;
+            constexpr bool F = decltype(fwd_tag)::value;
+            const uint32_t n = F ? nb.up[D] : nb.dn[D];
+            Su3<R> u;
+            V sp[12];
+            GaugeLoad<FMT>::load(a.gauge, S, D, F ? P : P ^ 1, F ? i : n, u);
+            load_spinor<R>(sp, in, S, n);
+            hop_rows<D, F>(t, sp, u, F ? Cx<R>{R(a.w.wf[D][0]), R(a.w.wf[D][1])} : Cx<R>{R(a.w.wb[D][0]), R(a.w.wb[D][1])});
+        };
+        switch (wave) {
+            case 0: hop(std::integral_constant<int, 0>{}, std::true_type{}); break;
+            case 1: hop(std::integral_constant<int, 0>{}, std::false_type{}); break;
+            case 2: hop(std::integral_constant<int, 1>{}, std::true_type{}); break;
+            case 3: hop(std::integral_constant<int, 1>{}, std::false_type{}); break;
+            case 4: hop(std::integral_constant<int, 2>{}, std::true_type{}); break;
+            case 5: hop(std::integral_constant<int, 2>{}, std::false_type{}); break;
+            case 6: hop(std::integral_constant<int, 3>{}, std::true_type{}); break;
+            default: hop(std::integral_constant<int, 3>{}, std::false_type{}); break;
+        }
+#pragma unroll
+        for (int k = 0; k < 6; ++k) rows[(wave * 6 + k) * SPLIT_SITES + lane] = V{t[k].re, t[k].im};
+    }
+    __syncthreads();
+    double nrm = 0., ry = 0.;
+    if (live && wave < 6) {
+        Cx<R> acc[2];
+        switch (wave) {
+            case 0: pair_sum<0>(acc, rows, lane); break;
+            case 1: pair_sum<1>(acc, rows, lane); break;
+            case 2: pair_sum<2>(acc, rows, lane); break;
+            case 3: pair_sum<3>(acc, rows, lane); break;
+            case 4: pair_sum<4>(acc, rows, lane); break;
+            default: pair_sum<5>(acc, rows, lane); break;
+        }
+        const bool upper = wave < 3;  // spins 0 and 1
+        const Cx<R> f    = upper ? Cx<R>{R(a.f1[0]), R(a.f1[1])} : Cx<R>{R(a.f2[0]), R(a.f2[1])};
+        if (a.epilogue == EPI_MINV) {
+            const R sc = R(a.scale);
+            acc[0]     = scale(cmul(acc[0], f), sc);
+            acc[1]     = scale(cmul(acc[1], f), sc);
+        } else if (a.epilogue == EPI_AEE) {
+            V x[2];
+            load_pair<R>(x, a.x, S, wave, i);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[j] = cmul(Cx<R>{x[j].x, x[j].y}, f) - acc[j];
+                if (a.gamma5 && !upper) acc[j] = Cx<R>{-acc[j].re, -acc[j].im};
+            }
+        }
+        if (a.cg_r) {  // the CG residual in place of the result, as CL2_FINISH_SITE
+            const Cx<R> al{R(a.cg_alpha[0]), R(a.cg_alpha[1])};
+            V ro[2];
+            load_pair<R>(ro, a.cg_r, S, wave, i);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[j] = Cx<R>{ro[j].x, ro[j].y} - cmul(acc[j], al);
+                ry += (double)acc[j].re * (double)ro[j].x + (double)acc[j].im * (double)ro[j].y;
+            }
+        }
+        if (a.norm_partials)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                nrm += (double)acc[j].re * (double)acc[j].re + (double)acc[j].im * (double)acc[j].im;
+        store_pair<R>(a.cg_r ? a.cg_r : a.out, S, wave, i, acc[0], acc[1]);
+    }
+    if (a.norm_partials) {
+        const double2 s = block_sum2<SPLIT_BLOCK>(make_double2(nrm, ry), lds);
+        if (threadIdx.x == 0) a.norm_partials[2 * blockIdx.x] = s.x, a.norm_partials[2 * blockIdx.x + 1] = s.y;
+    }
+}
+
 bool mrhs_offsets_narrow(uint32_t veo, int nrhs, size_t complex_bytes)
 {
     return (uint64_t)veo * (uint64_t)nrhs * complex_bytes <= 0xffffffffull;
@@ -534,6 +705,25 @@ __global__ __launch_bounds__(BLOCK) void k_sitediag(vec2<R>* __restrict__ out, c
     store_spinor<R>(out, S, i, v);
 }
 
+/* whether a lattice of veo eo sites takes the wave-per-hop kernel for links of format fmt (default shapes; one
+ * thread per site / wave per hop in us per dslash_eo, one run):
+ *   FP64  8^4 7.6 / 4.8, 12^3x20 11.7 / 9.0, 14^3x22 13.9 / 11.3, but 14^3x40 17.0 / 19.7, 16^3x32 19.3 / 20.9, where
+ *         the 256-thread blocks of the other kernel fill the chip and its fewer bytes in LDS count;
+ *   FP32  8^4 5.7 / 4.7, 14^3x22 7.7 / 5.1, 16^3x24 8.6 / 7.8, but 14^3x40 8.2 / 8.5, 16^3x32 9.5 / 9.8 (one block per
+ *         compute unit); beyond, as long as links and spinors fit the Infinity Cache, again 18^3x34 14.2 / 13.7,
+ *         20^3x40 21.6 / 19.5, 24^3x48 38.8 / 35.8, and then 28^3x56 69.0 / 69.8, 32^3x64 112 / 114;
+ *   FP16  8^4 5.0 / 4.8, 14^3x22 6.6 / 4.9, 14^3x40 6.9 / 6.5, 16^3x32 7.1 / 7.3, 20^3x40 12.9 / 13.8. */
+static bool wave_per_hop(int fmt, uint32_t veo)
+{
+    switch (fmt) {
+        case GAUGE_F64_18:
+        case GAUGE_F64_12: return veo <= 40000;
+        case GAUGE_F32_12: return veo <= 50000 || (veo >= 90000 && veo <= 400000);
+        case GAUGE_F16_12: return veo <= 60000;
+        default: return false;  // the staggered kernels have no such variant
+    }
+}
+
 cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs)
 {
     if (!c->tune_manual) {
@@ -545,7 +735,9 @@ cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs)
     const int occ = c->tune_occ >= 0
                         ? c->tune_occ
                         : ((fmt == GAUGE_F64_18 || fmt == GAUGE_F64_12) ? 1 : (fmt == GAUGE_F32_12 ? 2 : 0));
-    return cl2_hop_tuning{c->tune_zplanes, c->tune_xcd, c->tune_mrhs_rb, c->tune_mrhs_lds, c->tune_block, occ};
+    cl2_hop_tuning t{c->tune_zplanes, c->tune_xcd, c->tune_mrhs_rb, c->tune_mrhs_lds, c->tune_block, occ};
+    if (!c->tune_manual && nrhs == 1 && wave_per_hop(fmt, c->g.veo)) t.block = SPLIT_SITES;
+    return t;
 }
 
 WorkMap work_map(const cl2_ctx* c, int block, int nrhs, const cl2_hop_tuning& t)
@@ -647,6 +839,22 @@ static hipError_t launch_dslash_n(cl2_ctx* c, const DslashArgs& a, int format)
 {
     if constexpr (NRHS == 1) {
         if (format == GAUGE_F16_12) return launch_dslash_h(c, a);
+        if (a.block == SPLIT_SITES) {
+            const unsigned ns = blocks_for((size_t)a.g.veo, SPLIT_SITES);
+            switch (format) {
+                case GAUGE_F64_18:
+                    hipLaunchKernelGGL(k_dslash_eo_split<GAUGE_F64_18>, dim3(ns), dim3(SPLIT_BLOCK), 0, c->stream, a);
+                    break;
+                case GAUGE_F64_12:
+                    hipLaunchKernelGGL(k_dslash_eo_split<GAUGE_F64_12>, dim3(ns), dim3(SPLIT_BLOCK), 0, c->stream, a);
+                    break;
+                case GAUGE_F32_12:
+                    hipLaunchKernelGGL(k_dslash_eo_split<GAUGE_F32_12>, dim3(ns), dim3(SPLIT_BLOCK), 0, c->stream, a);
+                    break;
+                default: return hipErrorInvalidValue;
+            }
+            return hipGetLastError();
+        }
         auto by_shape = [&](auto fmt_tag) -> hipError_t {
             constexpr int F = decltype(fmt_tag)::value;
             const unsigned bs = (unsigned)a.block;

@@ -1,0 +1,175 @@
+"""The kernels that a rule on sizes picks, against the general ones, on the GPU.
+
+* the wave-per-hop hopping kernel of small lattices gives the bits of the thread-per-site kernel, for lattices that
+  do not fill a block of 64 sites or a link tile, plain, with the Aee epilogue and in the fused CG step;
+* the staggered multi-RHS kernel with two right-hand sides per thread gives the single-field kernel's bits where the
+  last block is not full, and fields that are not 16-byte aligned take the one-per-thread kernel;
+* MdagM_eo equals its two D_KS_eo and the elementwise saxpby bit for bit;
+* the streaming multi-shift update agrees with numpy;
+* stage 2 of the reductions sums every one of many partials once.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle as O
+from cl2qcd_amd import abi
+from fields import random_su3_field
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [(abi.GAUGE_F64_18, abi.F64), (abi.GAUGE_F64_12, abi.F64), (abi.GAUGE_F32_12, abi.F32),
+           (abi.GAUGE_F16_12, abi.F16)]
+KAPPA, MUBAR = 0.16, 0.0016
+
+
+@pytest.mark.parametrize("phases", [dict(theta_t=1.0), dict(theta_t=1.0, theta_s=0.3, cp_im=0.2)],
+                         ids=["real-spatial-weights", "complex-weights"])
+@pytest.mark.parametrize("ns,nt", [(2, 2), (6, 10), (8, 4)])  # 8, 1080 and 1024 eo sites
+@pytest.mark.parametrize("fmt,prec", FORMATS)
+def test_wave_per_hop_matches_thread_per_site(fmt, prec, ns, nt, phases):
+    lat = O.lattice(ns, nt, **phases)
+    results = []
+    for block in (None, 256):
+        with abi.Context(ns, nt, **phases) as ctx:
+            if block:
+                ctx.tune_set(b"hop.block", block)
+            rng = np.random.default_rng(7)
+            gf = ctx.gauge(random_su3_field(4 * O.volume(lat), 8), fmt)
+            src, r0 = rng.standard_normal((ctx.veo, 24)), rng.standard_normal((ctx.veo, 24))
+            a, b, r = ctx.spinor(prec).upload(src), ctx.spinor(prec), ctx.spinor(prec).upload(r0)
+            tmp = ctx.buffer(2 * ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SPINOR_EO, prec))
+            got = []
+            for evenodd in (abi.EVEN, abi.ODD):
+                ctx.dslash_eo(b.ptr, a.ptr, gf.ptr, fmt, evenodd, KAPPA)
+                got.append(b.download())
+            ctx.fermionmatrix_eo(abi.OP_AEE_MINUS_AND_GAMMA5, b.ptr, a.ptr, gf.ptr, fmt, abi.ACTION_TWISTEDMASS, KAPPA,
+                                 MUBAR, tmp.ptr)
+            got.append(b.download())
+            s = ctx.scalars(10)
+            s.store([O.norm2(r0)] + [0.0] * 9)
+            ctx.fermionmatrix_eo_cg_step(abi.OP_QPLUSQMINUS_EO, r.ptr, a.ptr, gf.ptr, fmt, abi.ACTION_TWISTEDMASS,
+                                         KAPPA, MUBAR, tmp.ptr, s.at(0), s.at(2), s.at(4), s.at(6))
+            results.append((got, r.download(), s.get()))
+    (got, res, sc), (ref, rres, rsc) = results
+    for x, y in zip(got, ref):
+        assert np.array_equal(x, y)
+    # the norms are the same terms grouped by component pairs: FP64 sums; for FP16 each group is a float chain of 4
+    # instead of 24 terms, 24 * 2^-24 relative
+    tol = 1.5e-6 if prec == abi.F16 else 1e-13
+    assert abs(sc[2] - rsc[2]) <= tol * rsc[2]
+    if prec == abi.F16:
+        # alpha follows pAp within tol; r_new is requantised to 2^-11 of the site's largest entry
+        assert np.abs(res - rres).max() <= 2.0 ** -10 * np.abs(rres).max()
+    else:
+        bound = 1e-12 if prec == abi.F64 else 4 * 2.0 ** -23
+        assert np.abs(res - rres).max() <= bound * np.abs(rres).max()
+    assert abs(sc[6] - rsc[6]) <= (2e-3 if prec == abi.F16 else 1e-6) * rsc[6]
+
+
+@pytest.mark.parametrize("nrhs", [8, 12, 16])
+@pytest.mark.parametrize("offset", [0, 8])
+def test_staggered_pairs_match_single(nrhs, offset):
+    ns, nt, mass = 6, 10, 0.1  # 1080 eo sites: 33 blocks of 32 sites and a rest of 24
+    with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        lat = O.lattice(ns, nt, theta_t=1.0)
+        gf = ctx.gauge(random_su3_field(4 * O.volume(lat), 3)).converted(abi.GAUGE_F32_12)
+        rng = np.random.default_rng(nrhs)
+        one = ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SU3VEC_EO, abi.F32)
+        blk, out = ctx.buffer(nrhs * one + 16), ctx.buffer(nrhs * one + 16)
+        bp, op = blk.ptr + offset, out.ptr + offset
+        src = [rng.standard_normal((ctx.veo, 6)) for _ in range(nrhs)]
+        a, b = ctx.su3vec(abi.F32), ctx.su3vec(abi.F32)
+        for r, v in enumerate(src):
+            ctx.block_insert_stagg_eo(bp, a.upload(v).ptr, abi.F32, nrhs, r)
+        for evenodd in (abi.EVEN, abi.ODD):
+            ctx.D_KS_eo_mrhs(op, bp, gf.ptr, abi.GAUGE_F32_12, evenodd, nrhs)
+            for r in range(nrhs):
+                ctx.D_KS_eo(b.ptr, a.upload(src[r]).ptr, gf.ptr, abi.GAUGE_F32_12, evenodd)
+                got = ctx.su3vec(abi.F32)
+                ctx.block_extract_stagg_eo(got.ptr, op, abi.F32, nrhs, r)
+                assert np.array_equal(got.download(), b.download())
+        # the fused step's sums: |D p|^2 + (m^2 + sigma) |p|^2 per right-hand side, against numpy
+        s = ctx.scalars(10 * nrhs)
+        s.store(np.concatenate([np.ones(2 * nrhs), np.zeros(8 * nrhs)]))
+        rb, tb = ctx.buffer(nrhs * one + 16), ctx.buffer(nrhs * one + 16)
+        sigma = (ctypes.c_double * nrhs)(*np.linspace(0.0, 1.0, nrhs))
+        ctx.MdagM_eo_mrhs_cg_step(rb.ptr + offset, bp, gf.ptr, abi.GAUGE_F32_12, mass, abi.EVEN, sigma, tb.ptr + offset,
+                                  nrhs, s.at(0), s.at(nrhs), s.at(2 * nrhs), s.at(4 * nrhs), s.at(6 * nrhs))
+        pap = s.get()[2 * nrhs:4 * nrhs:2]
+        for r in range(nrhs):
+            p = a.upload(src[r]).download()
+            ctx.D_KS_eo(b.ptr, a.ptr, gf.ptr, abi.GAUGE_F32_12, abi.ODD)
+            ref = (b.download() ** 2).sum() + (mass * mass + sigma[r]) * (p ** 2).sum()
+            assert abs(pap[r] - ref) <= 1e-12 * ref
+
+
+@pytest.mark.parametrize("fmt,prec", FORMATS[:3])
+def test_mdagm_is_two_hops_and_saxpby(fmt, prec):
+    ns, nt, mass = 6, 10, 0.37
+    with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        lat = O.lattice(ns, nt, theta_t=1.0)
+        gf = ctx.gauge(random_su3_field(4 * O.volume(lat), 4), fmt)
+        x = ctx.su3vec(prec).upload(np.random.default_rng(5).standard_normal((ctx.veo, 6)))
+        out, w, ref, tmp = (ctx.su3vec(prec) for _ in range(4))
+        for upper, first in ((abi.EVEN, abi.ODD), (abi.ODD, abi.EVEN)):
+            ctx.MdagM_eo(out.ptr, x.ptr, gf.ptr, fmt, mass, upper, tmp.ptr)
+            ctx.D_KS_eo(w.ptr, x.ptr, gf.ptr, fmt, first)
+            ctx.D_KS_eo(ref.ptr, w.ptr, gf.ptr, fmt, upper)
+            ctx.saxpby_stagg_eo(ref.ptr, x.ptr, ref.ptr, prec, abi.scalar(mass * mass), abi.scalar(-1.0))
+            assert np.array_equal(out.download(), ref.download())
+
+
+def test_streaming_multishift_update():
+    n = 60  # FP64 x and FP32 p of 16^3x32: 283 MB, above the 256 MiB where the update starts to stream
+    with abi.Context(16, 32) as ctx:
+        rng = np.random.default_rng(2)
+        r = ctx.su3vec(abi.F32).upload(rng.standard_normal((ctx.veo, 6)))
+        xs, ps = [], []
+        for k in range(n):
+            xs.append(ctx.su3vec(abi.F64))
+            ps.append(ctx.su3vec(abi.F32))
+            ctx.gaussian_eo(abi.FIELD_SU3VEC_EO, xs[k].ptr, abi.F64, 10 + k)
+            ctx.gaussian_eo(abi.FIELD_SU3VEC_EO, ps[k].ptr, abi.F32, 100 + k)
+        check = [0, 1, 31, 58, 59]
+        before = {k: (xs[k].download(), ps[k].download()) for k in check}
+        coef = rng.standard_normal((3, n))
+        active = np.ones(n)
+        active[[1, 58]] = 0.0
+        dev = ctx.scalars(4 * n)
+        dev.store(np.concatenate([coef.ravel(), active]))
+        ctx.multishift_update_stagg_eo((ctypes.c_void_p * n)(*[x.ptr for x in xs]), abi.F64,
+                                       (ctypes.c_void_p * n)(*[p.ptr for p in ps]), r.ptr, abi.F32, n, dev.at(0),
+                                       dev.at(n), dev.at(2 * n), dev.at(3 * n))
+        R = r.download()
+        for k in check:
+            x, p = before[k]
+            if active[k]:
+                x, p = coef[0, k] * p + x, coef[1, k] * R + coef[2, k] * p
+            # one product and one sum per element: two roundings of FP64 (x), of FP32 with rounded factors (p)
+            assert np.abs(xs[k].download() - x).max() <= 4 * 2.0 ** -53 * np.abs(x).max()
+            assert np.abs(ps[k].download() - p).max() <= 6 * 2.0 ** -24 * np.abs(p).max() + 1e-30
+
+
+def test_many_partial_sums():
+    # 8262 partials of 1024 elements: the second stage with eight loads in flight, and a rest of 70
+    with abi.Context(24, 102) as ctx:
+        f, s = ctx.spinor(abi.F64), ctx.scalars(2)
+        ctx.set_cold_eo(f.ptr, abi.F64)
+        ctx.squarenorm_eo(s.ptr, f.ptr, abi.F64)
+        assert abs(s.get()[0] - 0.5) < 1e-13  # every component is 1 / sqrt(12 V), V twice the eo sites
+    # the block form: 8194 partials per right-hand side (one per 32 sites)
+    with abi.Context(2, 65552) as ctx:
+        one = ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SU3VEC_EO, abi.F32)
+        gf = ctx.gauge(fmt=abi.GAUGE_F32_12, seed=1, epsilon=0.0)
+        p, r, t, s = ctx.buffer(2 * one), ctx.buffer(2 * one), ctx.buffer(2 * one), ctx.scalars(20)
+        s.store([1.0] * 4 + [0.0] * 16)
+        f = ctx.su3vec(abi.F32)
+        ctx.set_cold_stagg_eo(f.ptr, abi.F32)
+        for k in range(2):
+            ctx.block_insert_stagg_eo(p.ptr, f.ptr, abi.F32, 2, k)
+        ctx.MdagM_eo_mrhs_cg_step(r.ptr, p.ptr, gf.ptr, abi.GAUGE_F32_12, 1.0, abi.EVEN, None, t.ptr, 2, s.at(0), s.at(2),
+                                  s.at(4), s.at(8), s.at(12))
+        # unit links and a constant field: D_KS_eo cancels, so <p, A p> = |p|^2 = 1/2
+        assert np.abs(s.get()[4:8:2] - 0.5).max() < 1e-6
