@@ -233,7 +233,7 @@ int run_dslash(cl2_ctx* c, void* out, const void* in, const void* x, const void*
         CL2_REQUIRE(c, aligned16(out) && aligned16(x) && aligned16(cg_r),
                     "FP32 Wilson spinor fields must be 16-byte aligned");
     }
-    DslashArgs a;
+    DslashRhsArgs a;
     a.in            = in;
     a.out           = out;
     a.gauge         = gauge;
@@ -252,7 +252,7 @@ int run_dslash(cl2_ctx* c, void* out, const void* in, const void* x, const void*
     a.cg_alpha      = cg_alpha;
     a.per_rhs       = (pr != nullptr && nrhs > 1) ? 1 : 0;
     a.w             = wilson_weights(c, a.per_rhs ? 1.0 : kappa);
-    for (int r = 0; r < 16; ++r) {
+    for (int r = 0; nrhs > 1 && r < 16; ++r) {
         const bool use   = a.per_rhs && r < nrhs;
         a.rhs_kappa[r]   = use ? pr->kappa[r] : 0.;
         a.rhs_f1[r][0]   = use ? pr->f1[r][0] : 0.;

@@ -797,7 +797,7 @@ struct MrhsH {
 };
 
 template<int NRHS, bool RS>
-__global__ __launch_bounds__(MrhsH<NRHS>::BLOCK) void k_dslash_eo_mrhs_h(DslashArgs a)
+__global__ __launch_bounds__(MrhsH<NRHS>::BLOCK) void k_dslash_eo_mrhs_h(DslashRhsArgs a)
 {
     constexpr int SB        = MrhsH<NRHS>::SB;
     constexpr int BLOCK     = MrhsH<NRHS>::BLOCK;
@@ -912,7 +912,7 @@ __global__ __launch_bounds__(MrhsH<NRHS>::BLOCK) void k_dslash_eo_mrhs_h(DslashA
     }
 }
 
-hipError_t launch_dslash_mrhs_h(cl2_ctx* c, const DslashArgs& a)
+hipError_t launch_dslash_mrhs_h(cl2_ctx* c, const DslashRhsArgs& a)
 {
     const bool rs = spatial_weights_real(a.w);
     auto go = [&](auto n_tag) -> hipError_t {

@@ -79,7 +79,7 @@ bool supported_nrhs(int n);
 HopWeights<double> wilson_weights(const cl2_ctx* c, double kappa);
 
 /* launchers (return hipSuccess or the launch error) */
-hipError_t launch_dslash(cl2_ctx* c, const DslashArgs& a, int format);
+hipError_t launch_dslash(cl2_ctx* c, const DslashRhsArgs& a, int format);
 hipError_t launch_sitediag(cl2_ctx* c, void* out, const void* in, int prec, const double f1[2], const double f2[2],
                            double scale);
 /* with x: out = coef x - D in (the last step of MdagM_eo) */
@@ -152,7 +152,7 @@ hipError_t launch_sitediag_h(cl2_ctx* c, void* out, const void* in, const double
 hipError_t launch_fill_h(cl2_ctx* c, void* out, double re, double im, uint32_t sites = 0);
 hipError_t launch_convert_h(cl2_ctx* c, void* out, int out_prec, const void* in, int in_prec, uint32_t sites = 0);
 /* blocks of FP16 spinors: the multi-RHS hopping kernel and the block BLAS */
-hipError_t launch_dslash_mrhs_h(cl2_ctx* c, const DslashArgs& a);
+hipError_t launch_dslash_mrhs_h(cl2_ctx* c, const DslashRhsArgs& a);
 hipError_t launch_block_axpy_h(cl2_ctx* c, void* out, const void* x, const void* y, int nrhs, const double* coef,
                                double sign, double* norms);
 hipError_t launch_block_xp_h(cl2_ctx* c, void* x, void* p, const void* r, int nrhs, const double* alpha,

@@ -168,13 +168,15 @@ __device__ __forceinline__ void hop_pair(Cx<R> (&acc)[12], const vec2<R>* __rest
         const size_t o_ = (O);                                                                                    \
         Cx<R> f1{R(a.f1[0]), R(a.f1[1])}, f2{R(a.f2[0]), R(a.f2[1])};                                             \
         R s_ = R(a.scale);                                                                                        \
-        if (a.per_rhs) {                                                                                          \
-            const R kr = R(a.rhs_kappa[rhs]);                                                                     \
-            _Pragma("unroll") for (int k = 0; k < 12; ++k) acc[k] = scale(acc[k], kr);                            \
-            f1 = Cx<R>{R(a.rhs_f1[rhs][0]), R(a.rhs_f1[rhs][1])};                                                 \
-            f2 = Cx<R>{R(a.rhs_f2[rhs][0]), R(a.rhs_f2[rhs][1])};                                                 \
-            s_ = R(a.rhs_scale[rhs]);                                                                             \
-        }                                                                                                         \
+        if constexpr (NRHS > 1)                                                                                   \
+            if (a.per_rhs) {                                                                                      \
+                const R kr = R(a.rhs_kappa[rhs]);                                                                 \
+                _Pragma("unroll") for (int k = 0; k < 12; ++k) acc[k] = scale(acc[k], kr);                        \
+                f1 = Cx<R>{R(a.rhs_f1[rhs][0]), R(a.rhs_f1[rhs][1])};                                             \
+                f2 = Cx<R>{R(a.rhs_f2[rhs][0]), R(a.rhs_f2[rhs][1])};                                             \
+                s_ = R(a.rhs_scale[rhs]);                                                                         \
+            }                                                                                                     \
+                                                                                                               \
         if (a.epilogue == EPI_MINV) {                                                                             \
             _Pragma("unroll") for (int k = 0; k < 12; ++k) acc[k] = scale(cmul(acc[k], k < 6 ? f1 : f2), s_);    \
         } else if (a.epilogue == EPI_AEE) {                                                                       \
@@ -218,7 +220,7 @@ __device__ __forceinline__ void hop_pair(Cx<R> (&acc)[12], const vec2<R>* __rest
 template<int FMT, int BLOCK, int NRHS, int OCC = 0, bool PLAIN = false>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(OCC == 4 ? 4 : 1, OCC == 4 ? 8 : (OCC == 1 ? 1 : 2))))
-void k_dslash_eo(DslashArgs a)
+void k_dslash_eo(typename std::conditional<NRHS == 1, DslashArgs, DslashRhsArgs>::type a)
 {
     using R = typename GaugeLoad<FMT>::R;
     using V = vec2<R>;
@@ -466,7 +468,7 @@ struct MrhsLds {
  * This removes the per-lane index arithmetic, link loads and 12-real reconstruction that otherwise repeat
  * NRHS times per site.  Per right-hand side the arithmetic is the single-field kernel's, in the same order. */
 template<int FMT, int NRHS, int SBX, bool WIDE = false>
-__global__ __launch_bounds__((MrhsLds<NRHS, SBX>::BLOCK)) void k_dslash_eo_mrhs_lds(DslashArgs a)
+__global__ __launch_bounds__((MrhsLds<NRHS, SBX>::BLOCK)) void k_dslash_eo_mrhs_lds(DslashRhsArgs a)
 {
     using R = typename GaugeLoad<FMT>::R;
     using V = vec2<R>;
@@ -737,6 +739,10 @@ cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs)
                         : ((fmt == GAUGE_F64_18 || fmt == GAUGE_F64_12) ? 1 : (fmt == GAUGE_F32_12 ? 2 : 0));
     cl2_hop_tuning t{c->tune_zplanes, c->tune_xcd, c->tune_mrhs_rb, c->tune_mrhs_lds, c->tune_block, occ};
     if (!c->tune_manual && nrhs == 1 && wave_per_hop(fmt, c->g.veo)) t.block = SPLIT_SITES;
+    // Wilson fields that stay in the L2s anyway run in site order instead of slabs (slabs / site order, dslash_eo in
+    // us: FP64 16^3x32 19.4 / 18.6, 20^3x40 48.1 / 47.9; FP32 16^3x32 9.5 / 8.6; FP16 7.1 / 7.0, its operators 7.8 /
+    // 7.4; but FP64 24^3x48 94.5 / 96.4; the staggered and multi-RHS kernels are no faster that way)
+    if (!c->tune_manual && nrhs == 1 && !(fmt & DKS_TUNING_KEY) && c->g.veo <= 200000) t.zplanes = 0;
     return t;
 }
 
@@ -791,7 +797,7 @@ HopWeights<double> wilson_weights(const cl2_ctx* c, double kappa)
 }
 
 template<int FMT, int NRHS, int RB>
-static hipError_t launch_rb(cl2_ctx* c, const DslashArgs& a)
+static hipError_t launch_rb(cl2_ctx* c, const DslashRhsArgs& a)
 {
     const unsigned nb = blocks_for((size_t)a.g.veo * (NRHS / RB), DSLASH_BLOCK);
     // one right-hand side per thread: per-site LDS staging of links and neighbour indices, or the single-field
@@ -818,7 +824,7 @@ static hipError_t launch_rb(cl2_ctx* c, const DslashArgs& a)
         }
     } else
         hipLaunchKernelGGL((k_dslash_eo_rb<FMT, DSLASH_BLOCK, NRHS, RB>), dim3(nb), dim3(DSLASH_BLOCK), 0, c->stream,
-                           a);
+                           static_cast<const DslashArgs&>(a));
     return hipGetLastError();
 }
 
@@ -835,8 +841,10 @@ static int rhs_per_thread(const DslashArgs& a)
 }
 
 template<int NRHS>
-static hipError_t launch_dslash_n(cl2_ctx* c, const DslashArgs& a, int format)
+static hipError_t launch_dslash_n(cl2_ctx* c, const DslashRhsArgs& ra, int format)
 {
+    // single-field kernels take the short argument block
+    const typename std::conditional<NRHS == 1, DslashArgs, DslashRhsArgs>::type& a = ra;
     if constexpr (NRHS == 1) {
         if (format == GAUGE_F16_12) return launch_dslash_h(c, a);
         if (a.block == SPLIT_SITES) {
@@ -938,7 +946,7 @@ bool supported_nrhs(int n)
     return n == 1 || n == 2 || n == 4 || n == 8 || n == 12 || n == 16;
 }
 
-hipError_t launch_dslash(cl2_ctx* c, const DslashArgs& a, int format)
+hipError_t launch_dslash(cl2_ctx* c, const DslashRhsArgs& a, int format)
 {
     switch (a.nrhs) {
         case 1: return launch_dslash_n<1>(c, a, format);
