@@ -218,7 +218,7 @@ struct RhsParams {
 int run_dslash(cl2_ctx* c, void* out, const void* in, const void* x, const void* gauge, int fmt, int evenodd,
                double kappa, int epilogue, const double f1[2], const double f2[2], double scale, int gamma5,
                int nrhs = 1, const RhsParams* pr = nullptr, double* norm_res = nullptr, void* cg_r = nullptr,
-               const double* cg_alpha = nullptr)
+               const double* cg_alpha = nullptr, const SumTail* tail = nullptr)
 {
     CL2_REQUIRE(c, valid_fmt(fmt), "unknown gauge format");
     CL2_REQUIRE(c, supported_nrhs(nrhs), "unsupported number of right-hand sides (1, 2, 4, 8, 12 or 16)");
@@ -292,11 +292,12 @@ int run_dslash(cl2_ctx* c, void* out, const void* in, const void* x, const void*
     // complex (norm, 0), or with the CG update (|r_new|^2, Re <r_new, r_old>, |r_new|^2, 0); the staged
     // multi-RHS kernel writes (|out|^2 or |r_new|^2, 0 or Re <r_new, r_old>) per right-hand side and block
     if (norm_res && !mrhs_norms)
-        CL2_HIP(c, launch_reduce_stage2(c, blocks_for(a.g.veo, a.block), norm_res, cg_r ? 3 : 1, nullptr, 0));
+        CL2_HIP(c, launch_reduce_stage2(c, blocks_for(a.g.veo, a.block), norm_res, cg_r ? 3 : 1, nullptr, 0, nullptr,
+                                        tail));
     if (mrhs_norms) {
         const int sb = mrhs_sites_per_block(nrhs, a.lds);
         CL2_HIP(c, launch_block_reduce2(c, reinterpret_cast<const double2*>(c->partials),
-                                        (unsigned)((a.g.veo + sb - 1) / sb), norm_res, 0, nrhs));
+                                        (unsigned)((a.g.veo + sb - 1) / sb), norm_res, 0, nrhs, tail));
     }
     return CL2_OK;
 }
@@ -334,7 +335,7 @@ void tm_factors(int variant, double mubar, double f1[2], double f2[2], double* s
 int run_aee(cl2_ctx* c, void* out, const void* in, void* tmp, const void* gauge, int fmt, int action, double kappa,
             double mubar, bool minus, bool gamma5, int nrhs = 1, const double* kappas = nullptr,
             const double* mubars = nullptr, double* norm_res = nullptr, void* cg_r = nullptr,
-            const double* cg_alpha = nullptr)
+            const double* cg_alpha = nullptr, const SumTail* tail = nullptr)
 {
     double f1[2], f2[2], s;
     int rc;
@@ -361,21 +362,21 @@ int run_aee(cl2_ctx* c, void* out, const void* in, void* tmp, const void* gauge,
         rc = run_dslash(c, tmp, in, nullptr, gauge, fmt, CL2_ODD, 1., EPI_MINV, one, one, 1., 0, nrhs, &p1);
         if (rc) return rc;
         return run_dslash(c, out, tmp, in, gauge, fmt, CL2_EVEN, 1., EPI_AEE, one, one, 1., gamma5 ? 1 : 0, nrhs, &p2,
-                          norm_res, cg_r, cg_alpha);
+                          norm_res, cg_r, cg_alpha, tail);
     }
     if (action == CL2_ACTION_WILSON) {
         const double one[2] = {1., 0.};
         rc = run_dslash(c, tmp, in, nullptr, gauge, fmt, CL2_ODD, kappa, EPI_PLAIN, one, one, 1., 0, nrhs);
         if (rc) return rc;
         return run_dslash(c, out, tmp, in, gauge, fmt, CL2_EVEN, kappa, EPI_AEE, one, one, 1., gamma5 ? 1 : 0, nrhs,
-                          nullptr, norm_res, cg_r, cg_alpha);
+                          nullptr, norm_res, cg_r, cg_alpha, tail);
     }
     tm_factors(minus ? CL2_MTM_INVERSE_SITEDIAGONAL_MINUS : CL2_MTM_INVERSE_SITEDIAGONAL, mubar, f1, f2, &s);
     rc = run_dslash(c, tmp, in, nullptr, gauge, fmt, CL2_ODD, kappa, EPI_MINV, f1, f2, s, 0, nrhs);
     if (rc) return rc;
     tm_factors(minus ? CL2_MTM_SITEDIAGONAL_MINUS : CL2_MTM_SITEDIAGONAL, mubar, f1, f2, &s);
     return run_dslash(c, out, tmp, in, gauge, fmt, CL2_EVEN, kappa, EPI_AEE, f1, f2, 1., gamma5 ? 1 : 0, nrhs, nullptr,
-                      norm_res, cg_r, cg_alpha);
+                      norm_res, cg_r, cg_alpha, tail);
 }
 
 /* the eo operators on nrhs right-hand sides ([12][Veo][nrhs] fields, tmp = 2 such fields) */
@@ -920,10 +921,15 @@ int cl2_fermionmatrix_eo_cg_step(cl2_ctx* c, int op, void* r, const void* p, con
     void* t0        = tmp;
     void* t1        = static_cast<char*>(tmp) + fb;
     CL2_REQUIRE(c, r != t0 && r != t1 && p != t0 && p != t1, "tmp must not alias r or p");
-    // t1 = Qminus p with pAp = |t1|^2; alpha = r2 / pAp; then Qplus t1 is folded into r <- r - alpha Qplus t1
-    if (int rc = run_aee(c, t1, p, t0, gauge, fmt, action, kappa, mubar, true, true, 1, nullptr, nullptr, pAp))
+    // t1 = Qminus p with pAp = |t1|^2 and alpha = r2 / pAp by the block that finishes that sum; then Qplus t1 is folded
+    // into r <- r - alpha Qplus t1
+    SumTail tail{};
+    tail.kind  = TAIL_RATIO;
+    tail.r2    = r2;
+    tail.alpha = alpha;
+    if (int rc = run_aee(c, t1, p, t0, gauge, fmt, action, kappa, mubar, true, true, 1, nullptr, nullptr, pAp, nullptr,
+                         nullptr, &tail))
         return rc;
-    CL2_HIP(c, launch_scalar_op(c, CL2_SCALAR_OP_RATIO, 1, alpha, r2, pAp));
     return run_aee(c, nullptr, t1, t0, gauge, fmt, action, kappa, mubar, false, true, 1, nullptr, nullptr, norms, r,
                    alpha);
 }
@@ -947,9 +953,14 @@ int cl2_fermionmatrix_eo_mrhs_cg_step(cl2_ctx* c, int op, void* r, const void* p
     void* t0        = tmp;
     void* t1        = static_cast<char*>(tmp) + fb;
     CL2_REQUIRE(c, r != t0 && r != t1 && p != t0 && p != t1, "tmp must not alias r or p");
-    if (int rc = run_aee(c, t1, p, t0, gauge, fmt, action, kappa, mubar, true, true, nrhs, kappas, mubars, pAp))
+    SumTail tail{};
+    tail.kind   = TAIL_ALPHA;
+    tail.r2     = r2;
+    tail.active = active;
+    tail.alpha  = alpha;
+    if (int rc = run_aee(c, t1, p, t0, gauge, fmt, action, kappa, mubar, true, true, nrhs, kappas, mubars, pAp, nullptr,
+                         nullptr, &tail))
         return rc;
-    CL2_HIP(c, launch_block_cg_scalars(c, 0, alpha, const_cast<double*>(r2), pAp, active, nrhs));
     return run_aee(c, nullptr, t1, t0, gauge, fmt, action, kappa, mubar, false, true, nrhs, kappas, mubars, norms, r,
                    alpha);
 }
@@ -1377,16 +1388,19 @@ int cl2_MdagM_eo_mrhs_cg_step(cl2_ctx* c, void* r, const void* p, const void* ga
     CL2_REQUIRE(c, upper_left == CL2_EVEN || upper_left == CL2_ODD, "upper_left must be CL2_EVEN or CL2_ODD");
     CL2_REQUIRE(c, r && p && gauge && tmp && r2 && active && pAp && alpha && norms, "null pointer");
     CL2_REQUIRE(c, r != p && tmp != p && tmp != r, "r, p and tmp must be different blocks");
-    double coef[16];
-    for (int k = 0; k < nrhs; ++k) coef[k] = mass * mass + (sigma ? sigma[k] : 0.);
+    SumTail tail{};
+    tail.kind   = TAIL_ALPHA_MDAGM;
+    tail.r2     = r2;
+    tail.active = active;
+    tail.alpha  = alpha;
+    for (int k = 0; k < nrhs; ++k) tail.coef[k] = mass * mass + (sigma ? sigma[k] : 0.);
     const int first = (upper_left == CL2_EVEN) ? CL2_ODD : CL2_EVEN;
     double2* parts  = reinterpret_cast<double2*>(c->partials);
     unsigned nb     = 0;
     // w = D_KS p with per-right-hand-side (|w|^2, |p|^2); pAp and alpha on the device; then r -= alpha (coef p - D w)
     CL2_HIP(c, launch_dks_mrhs(c, tmp, p, gauge, fmt, first, nrhs, nullptr, nullptr, parts, p, nullptr, nullptr, &nb));
-    CL2_HIP(c, launch_block_reduce2(c, parts, nb, pAp, 0, nrhs));
-    CL2_HIP(c, launch_block_cg_alpha_mdagm(c, alpha, r2, pAp, coef, active, nrhs));
-    CL2_HIP(c, launch_dks_mrhs(c, nullptr, tmp, gauge, fmt, upper_left, nrhs, p, coef, parts, nullptr, r, alpha, &nb));
+    CL2_HIP(c, launch_block_reduce2(c, parts, nb, pAp, 0, nrhs, &tail));
+    CL2_HIP(c, launch_dks_mrhs(c, nullptr, tmp, gauge, fmt, upper_left, nrhs, p, tail.coef, parts, nullptr, r, alpha, &nb));
     CL2_HIP(c, launch_block_reduce2(c, parts, nb, norms, 0, nrhs));
     return CL2_OK;
 }
@@ -1635,8 +1649,14 @@ int cl2_MdagM_eo_cgm_step(cl2_ctx* c, void* r, const void* p, const void* gauge,
     unsigned nb     = 0;
     double* wp      = c->dscratch + 2;  // (|D p|^2, |p|^2)
     CL2_HIP(c, launch_dks_step(c, tmp, p, gauge, fmt, first, p, nullptr, 0., nullptr, nullptr, &nb));
-    CL2_HIP(c, launch_reduce_stage2(c, nb, wp, 1, nullptr, 0));
-    CL2_HIP(c, launch_cgm_beta_step_mdagm(c, beta, beta_prev, rr_old, pap, wp, m2));
+    SumTail tail{};
+    tail.kind      = TAIL_CGM_BETA;
+    tail.r2        = rr_old;
+    tail.beta      = beta;
+    tail.beta_prev = beta_prev;
+    tail.pap       = pap;
+    tail.m2        = m2;
+    CL2_HIP(c, launch_reduce_stage2(c, nb, wp, 1, nullptr, 0, nullptr, &tail));
     CL2_HIP(c, launch_dks_step(c, nullptr, tmp, gauge, fmt, upper_left, nullptr, p, m2, r, beta, &nb));
     CL2_HIP(c, launch_reduce_stage2(c, nb, rr_new, 0, nullptr, 0));
     return CL2_OK;

@@ -8,6 +8,8 @@
 // so results are reproducible run to run.
 #include <algorithm>
 
+#include <type_traits>
+
 #include "cl2_device.hpp"
 #include "cl2_internal.hpp"
 
@@ -249,10 +251,10 @@ hipError_t launch_reduce_stage1(cl2_ctx* c, const void* x, const void* y, size_t
 /* stage 2: one block sums the partials in a fixed order.
  * out_kind 0: res[0] = re;  1: res = (re, im);  2: res[k] = alpha[k]^2 * re for k < nvec;
  * 3: res = (re, im, re, 0) */
-template<int BLOCK, bool WIDE>
-__global__ __launch_bounds__(BLOCK) void k_reduce2(const double* __restrict__ partials, unsigned nparts,
-                                                   double* __restrict__ res, int out_kind,
-                                                   const double* __restrict__ alpha, int nvec)
+template<int BLOCK, bool WIDE, bool TAIL>
+__global__ __launch_bounds__(BLOCK) void k_reduce2(const double* __restrict__ partials, unsigned nparts, double* res,
+                                                   int out_kind, const double* __restrict__ alpha, int nvec,
+                                                   typename std::conditional<TAIL, SumTail, NoTail>::type tail)
 {
     __shared__ double lds[2 * BLOCK / 64];
     const double2 s =
@@ -271,20 +273,34 @@ __global__ __launch_bounds__(BLOCK) void k_reduce2(const double* __restrict__ pa
         } else {
             for (int k = 0; k < nvec; ++k) res[k] = alpha[k] * alpha[k] * s.x;
         }
+        if constexpr (TAIL) {
+            if (tail.kind == TAIL_RATIO) {
+                const double2 q = complex_ratio(tail.r2[0], tail.r2[1], s.x, s.y);
+                tail.alpha[0]   = q.x;
+                tail.alpha[1]   = q.y;
+            } else {  // TAIL_CGM_BETA, from (|D p|^2, |p|^2)
+                const double a    = tail.m2 * s.y + s.x;
+                tail.pap[0]       = a;
+                const double b    = tail.beta[0];
+                tail.beta_prev[0] = b;
+                tail.beta[0]      = 0.0 - tail.r2[0] / a;
+            }
+        }
     }
 }
 
 hipError_t launch_reduce_stage2(cl2_ctx* c, unsigned nparts, double* res, int out_kind, const double* alpha_vec,
-                                int nvec, const double* parts)
+                                int nvec, const double* parts, const SumTail* tail)
 {
     // 1024 threads: the elementwise kernels leave up to BLAS_MAX_BLOCKS partials
     const double* p = parts ? parts : c->partials;
+    auto go         = [&](auto kernel, auto t) {
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, c->stream, p, nparts, res, out_kind, alpha_vec, nvec, t);
+    };
     if (nparts >= WIDE_SUM_MIN(1024))
-        hipLaunchKernelGGL((k_reduce2<1024, true>), dim3(1), dim3(1024), 0, c->stream, p, nparts, res, out_kind,
-                           alpha_vec, nvec);
+        tail ? go(k_reduce2<1024, true, true>, *tail) : go(k_reduce2<1024, true, false>, NoTail{});
     else
-        hipLaunchKernelGGL((k_reduce2<1024, false>), dim3(1), dim3(1024), 0, c->stream, p, nparts, res, out_kind,
-                           alpha_vec, nvec);
+        tail ? go(k_reduce2<1024, false, true>, *tail) : go(k_reduce2<1024, false, false>, NoTail{});
     return hipGetLastError();
 }
 
@@ -463,9 +479,9 @@ __global__ void k_scalar_op(int op, int is_complex, double* out, const double* a
             ri = ar * bi + ai * br;
             break;
         case CL2_SCALAR_OP_RATIO: {
-            double nrm = br * br + bi * bi;
-            rr         = (ar * br + ai * bi) / nrm;
-            ri         = (ai * br - ar * bi) / nrm;
+            const double2 q = complex_ratio(ar, ai, br, bi);
+            rr              = q.x;
+            ri              = q.y;
             break;
         }
         case CL2_SCALAR_OP_SUM:
@@ -575,25 +591,6 @@ __global__ __launch_bounds__(64) void k_cgm_alpha_step(int numeq, double* alpha,
         alpha[0]      = a_new;
         rr_old[0]     = rn;
     }
-}
-
-/* the beta step from the fused MdagM step's sums: pap = m2 |p|^2 + |D p|^2 from wp = (|D p|^2, |p|^2) */
-__global__ void k_cgm_beta_step_mdagm(double* beta, double* beta_prev, const double* rr, double* pap, const double* wp,
-                                      double m2)
-{
-    if (threadIdx.x != 0) return;
-    const double a = m2 * wp[1] + wp[0];
-    pap[0]         = a;
-    const double b = beta[0];
-    beta_prev[0]   = b;
-    beta[0]        = 0.0 - rr[0] / a;
-}
-
-hipError_t launch_cgm_beta_step_mdagm(cl2_ctx* c, double* beta, double* beta_prev, const double* rr, double* pap,
-                                      const double* wp, double m2)
-{
-    hipLaunchKernelGGL(k_cgm_beta_step_mdagm, dim3(1), dim3(64), 0, c->stream, beta, beta_prev, rr, pap, wp, m2);
-    return hipGetLastError();
 }
 
 hipError_t launch_cgm_beta_step(cl2_ctx* c, double* beta, double* beta_prev, const double* rr, const double* pap)

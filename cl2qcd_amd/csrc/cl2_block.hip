@@ -10,6 +10,8 @@
 // stage 2 reduces each right-hand side's block partials with one block each.
 #include <initializer_list>
 
+#include <type_traits>
+
 #include "cl2_device.hpp"
 #include "cl2_internal.hpp"
 
@@ -228,18 +230,31 @@ __global__ __launch_bounds__(256) void k_block_dot(const void* x, const void* y,
 
 /* stage 2: block r sums right-hand side r's nb partials; out_kind 0: res[2r..2r+1] = complex sum,
  * 1: res[r] = real part */
-template<int BLOCK, bool WIDE>
+template<int BLOCK, bool WIDE, bool TAIL>
 __global__ __launch_bounds__(BLOCK) void k_block_reduce2(const double2* partials, unsigned nb, double* res,
-                                                         int out_kind)
+                                                         int out_kind,
+                                                         typename std::conditional<TAIL, SumTail, NoTail>::type tail)
 {
     __shared__ double lds[2 * BLOCK / 64];
     const double2 s = block_sum2<BLOCK>(strided_sum<BLOCK, WIDE>(partials + (size_t)blockIdx.x * nb, nb), lds);
     if (threadIdx.x == 0) {
+        const unsigned r = blockIdx.x;
+        double2 v        = s;
+        if constexpr (TAIL) {
+            // (|D p_r|^2, |p_r|^2) -> <p_r, (m^2 + sigma_r - D D) p_r> (D_KS anti-hermitian)
+            if (tail.kind == TAIL_ALPHA_MDAGM) v = make_double2(tail.coef[r] * s.y + s.x, 0.);
+            double2 al = make_double2(0., 0.);
+            if (tail.active[r] != 0.)
+                al = tail.kind == TAIL_ALPHA ? block_alpha(tail.r2[r], v.x, v.y)
+                                             : make_double2(tail.r2[r] * v.x / (v.x * v.x), 0.);
+            tail.alpha[2 * r]     = al.x;
+            tail.alpha[2 * r + 1] = al.y;
+        }
         if (out_kind == 0) {
-            res[2 * blockIdx.x]     = s.x;
-            res[2 * blockIdx.x + 1] = s.y;
+            res[2 * r]     = v.x;
+            res[2 * r + 1] = v.y;
         } else {
-            res[blockIdx.x] = s.x;
+            res[r] = v.x;
         }
     }
 }
@@ -265,41 +280,12 @@ __global__ void k_block_cg_alpha(double* alpha, const double* r2, const double* 
     if (r >= nrhs) return;
     double ar = 0., ai = 0.;
     if (active[r] != 0.) {
-        const double a = pAp[2 * r], b = pAp[2 * r + 1], d = a * a + b * b;
-        ar = r2[r] * a / d;
-        ai = -r2[r] * b / d;
+        const double2 al = block_alpha(r2[r], pAp[2 * r], pAp[2 * r + 1]);
+        ar               = al.x;
+        ai               = al.y;
     }
     alpha[2 * r]     = ar;
     alpha[2 * r + 1] = ai;
-}
-
-/* the staggered fused CG step: pAp holds (|D p_r|^2, |p_r|^2) per right-hand side on entry and the complex
- * <p_r, (m^2 + sigma_r - D D) p_r> = coef_r |p_r|^2 + |D p_r|^2 (D_KS anti-hermitian) on exit; then alpha as
- * k_block_cg_alpha */
-struct Coef16 {
-    double v[16];
-};
-__global__ void k_block_cg_alpha_mdagm(double* alpha, const double* r2, double* pAp, Coef16 coef, const double* active,
-                                       int nrhs)
-{
-    const int r = threadIdx.x;
-    if (r >= nrhs) return;
-    const double a = coef.v[r] * pAp[2 * r + 1] + pAp[2 * r];
-    pAp[2 * r]     = a;
-    pAp[2 * r + 1] = 0.;
-    double ar = 0.;
-    if (active[r] != 0.) ar = r2[r] * a / (a * a);
-    alpha[2 * r]     = ar;
-    alpha[2 * r + 1] = 0.;
-}
-
-hipError_t launch_block_cg_alpha_mdagm(cl2_ctx* c, double* alpha, const double* r2, double* pAp, const double* coef,
-                                       const double* active, int nrhs)
-{
-    Coef16 k{};
-    for (int r = 0; r < nrhs && r < 16; ++r) k.v[r] = coef[r];
-    hipLaunchKernelGGL(k_block_cg_alpha_mdagm, dim3(1), dim3(64), 0, c->stream, alpha, r2, pAp, k, active, nrhs);
-    return hipGetLastError();
 }
 
 /* beta_r = Polak-Ribiere <r_new, r_new - r_old> / |r_old|^2 (Fletcher-Reeves when that is negative) for
@@ -388,14 +374,16 @@ static BlockShape block_shape(cl2_ctx* c, size_t n, int prec, int nrhs, int u, b
 
 constexpr int BLOCK_U_REDUCE = 4;
 
-hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, double* res, int out_kind, int nrhs)
+hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, double* res, int out_kind, int nrhs,
+                                const SumTail* tail)
 {
+    auto go = [&](auto kernel, auto t) {
+        hipLaunchKernelGGL(kernel, dim3(nrhs), dim3(1024), 0, c->stream, parts, nb, res, out_kind, t);
+    };
     if (nb >= WIDE_SUM_MIN(1024))
-        hipLaunchKernelGGL((k_block_reduce2<1024, true>), dim3(nrhs), dim3(1024), 0, c->stream, parts, nb, res,
-                           out_kind);
+        tail ? go(k_block_reduce2<1024, true, true>, *tail) : go(k_block_reduce2<1024, true, false>, NoTail{});
     else
-        hipLaunchKernelGGL((k_block_reduce2<1024, false>), dim3(nrhs), dim3(1024), 0, c->stream, parts, nb, res,
-                           out_kind);
+        tail ? go(k_block_reduce2<1024, false, true>, *tail) : go(k_block_reduce2<1024, false, false>, NoTail{});
     return hipGetLastError();
 }
 

@@ -612,4 +612,17 @@ __device__ __forceinline__ double2 strided_sum(const double2* __restrict__ p, un
     return acc[0];
 }
 
+/* a / b of complex scalars (common_header_files/operations_complex.hpp:59-66) and the step length of one right-hand
+ * side of a lockstep CG */
+__device__ __forceinline__ double2 complex_ratio(double ar, double ai, double br, double bi)
+{
+    const double nrm = br * br + bi * bi;
+    return make_double2((ar * br + ai * bi) / nrm, (ai * br - ar * bi) / nrm);
+}
+__device__ __forceinline__ double2 block_alpha(double r2, double a, double b)
+{
+    const double d = a * a + b * b;
+    return make_double2(r2 * a / d, -r2 * b / d);
+}
+
 }  // namespace cl2

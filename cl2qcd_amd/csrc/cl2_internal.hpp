@@ -127,11 +127,30 @@ hipError_t launch_reduce_stage1(cl2_ctx* c, const void* x, const void* y, size_t
                                 unsigned* nblocks, double* parts = nullptr);
 /* partials launch_reduce_stage1 writes for these operands (at most BLAS_MAX_BLOCKS) */
 unsigned reduce_stage1_blocks(size_t n, int prec, const void* x, const void* y);
+/* scalar work that the block finishing a stage-2 sum does with it, instead of a launch of its own:
+ *   TAIL_RATIO       alpha = r2 / sum (complex scalars, as cl2_complex_op's ratio);
+ *   TAIL_CGM_BETA    pap = m2 sum.y + sum.x; beta_prev = beta; beta = 0 - r2 / pap (the CG-M step on MdagM_eo);
+ *   TAIL_ALPHA       per right-hand side: alpha = r2 / sum where active, else 0 (cl2_block_cg_alpha);
+ *   TAIL_ALPHA_MDAGM the same with sum replaced by coef sum.y + sum.x, also left in its place (the lockstep step on
+ *                    MdagM_eo + sigma) */
+enum SumTailKind : int { TAIL_RATIO = 1, TAIL_CGM_BETA = 2, TAIL_ALPHA = 3, TAIL_ALPHA_MDAGM = 4 };
+struct SumTail {
+    int kind;
+    const double* r2;
+    const double* active;
+    double* alpha;
+    double *beta, *beta_prev, *pap;
+    double m2;
+    double coef[16];
+};
+struct NoTail {
+};
+
 /* stage 2: sum nparts double2 partials in fixed order.  out_kind 0: res[0] = real part;
  * 1: res[0..1] = complex sum;  2: res[k] = alpha_vec[k]^2 * real part for k < nvec;
  * 3: res[0..3] = (re, im, re, 0) */
 hipError_t launch_reduce_stage2(cl2_ctx* c, unsigned nparts, double* res, int out_kind, const double* alpha_vec,
-                                int nvec, const double* parts = nullptr);
+                                int nvec, const double* parts = nullptr, const SumTail* tail = nullptr);
 
 hipError_t launch_gauge_update(cl2_ctx* c, void* gauge, double beta, int mode, uint64_t key);
 hipError_t launch_plaquette(cl2_ctx* c, const void* gauge, double* res);
@@ -169,7 +188,8 @@ hipError_t launch_block_dot(cl2_ctx* c, double* res, const void* x, const void* 
                             int ncomp = 12);
 /* stage 2 of the per-right-hand-side reductions: block r sums partials[r * nb .. r * nb + nb) in order;
  * out_kind 0: res[2r..2r+1] = complex sum, 1: res[r] = real part */
-hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, double* res, int out_kind, int nrhs);
+hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, double* res, int out_kind, int nrhs,
+                                const SumTail* tail = nullptr);
 hipError_t launch_block_xp(cl2_ctx* c, void* x, void* p, const void* r, int prec, int nrhs, const double* alpha,
                            const double* beta, int ncomp = 12);
 hipError_t launch_block_slot(cl2_ctx* c, void* block, const void* single_in, void* single_out, int prec, int nrhs,
@@ -178,8 +198,6 @@ hipError_t launch_scalar_copy(cl2_ctx* c, double* dst, const double* src, int n)
 hipError_t launch_cg_beta(cl2_ctx* c, double* mbeta, double* r2, const double* norms);
 hipError_t launch_block_cg_scalars(cl2_ctx* c, int which, double* out, double* r2, const double* in,
                                    const double* active, int nrhs);
-hipError_t launch_block_cg_alpha_mdagm(cl2_ctx* c, double* alpha, const double* r2, double* pAp, const double* coef,
-                                       const double* active, int nrhs);
 
 /* fused multi-shift CG vector update over n complex elements */
 hipError_t launch_multishift(cl2_ctx* c, void* const* xs_dev, int x_prec, void* const* ps_dev, const void* r, int prec,
@@ -191,8 +209,6 @@ hipError_t launch_vec_element(cl2_ctx* c, double* out, const double* in, int out
 hipError_t launch_cgm_update(cl2_ctx* c, int which, double* out, const double* a, const double* b, const double* d,
                              const double* e, const double* f, const double* g, int numeq);
 hipError_t launch_cgm_beta_step(cl2_ctx* c, double* beta, double* beta_prev, const double* rr, const double* pap);
-hipError_t launch_cgm_beta_step_mdagm(cl2_ctx* c, double* beta, double* beta_prev, const double* rr, double* pap,
-                                      const double* wp, double m2);
 hipError_t launch_cgm_alpha_step(cl2_ctx* c, int numeq, double* alpha, double* alpha_prev, const double* rr_new,
                                  double* rr_old, const double* beta, const double* beta_prev, const double* sigma,
                                  double* zeta, double* zeta_prev, double* zeta_foll, double* beta_vec,
