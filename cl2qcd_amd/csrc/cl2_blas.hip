@@ -508,6 +508,20 @@ __global__ void k_vec_element(double* out, const double* in, int out_index, int 
     if (threadIdx.x == 0) out[out_index] = in[in_index];
 }
 
+__global__ __launch_bounds__(cl2_mailbox::SIZE) void k_mail(cl2_mailbox* m, const double* src, int n, uint64_t number)
+{
+    if ((int)threadIdx.x < n) m->value[threadIdx.x] = src[threadIdx.x];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(&m->number, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+hipError_t launch_mail(cl2_ctx* c, const double* src, int n, uint64_t number)
+{
+    hipLaunchKernelGGL(k_mail, dim3(1), dim3(cl2_mailbox::SIZE), 0, c->stream, c->mail, src, n, number);
+    return hipGetLastError();
+}
+
 hipError_t launch_vec_element(cl2_ctx* c, double* out, const double* in, int out_index, int in_index)
 {
     hipLaunchKernelGGL(k_vec_element, dim3(1), dim3(64), 0, c->stream, out, in, out_index, in_index);

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -21,6 +22,13 @@ struct cl2_hop_tuning {
                   // four hops in flight), 4 (>= 4 waves, one hop at a time); -1: the format's default
 };
 
+/* scalars on their way to the host: the values, then the number of the transfer they belong to */
+struct cl2_mailbox {
+    static constexpr int SIZE = 64;
+    double value[SIZE];
+    uint64_t number;
+};
+
 struct cl2_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -31,6 +39,8 @@ struct cl2_ctx {
     double* partials = nullptr;  // reduction scratch: one double2 per block
     size_t npartials = 0;
     double* dscratch = nullptr;  // a few device doubles for host-read results
+    cl2_mailbox* mail = nullptr; // pinned host memory that a kernel writes scalars into (cl2_scalar_get)
+    std::mutex mail_mutex;       // one reader of the mailbox at a time
     void** ptr_table = nullptr;  // device copy of the field-pointer table of the multi-shift update (2 x 64)
     std::vector<void*> ptr_table_host;  // what ptr_table holds
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
@@ -195,6 +205,8 @@ hipError_t launch_block_xp(cl2_ctx* c, void* x, void* p, const void* r, int prec
 hipError_t launch_block_slot(cl2_ctx* c, void* block, const void* single_in, void* single_out, int prec, int nrhs,
                              int r, int ncomp = 12);
 hipError_t launch_scalar_copy(cl2_ctx* c, double* dst, const double* src, int n);
+/* n <= cl2_mailbox::SIZE doubles into the context's mailbox, then its number */
+hipError_t launch_mail(cl2_ctx* c, const double* src, int n, uint64_t number);
 hipError_t launch_cg_beta(cl2_ctx* c, double* mbeta, double* r2, const double* norms);
 hipError_t launch_block_cg_scalars(cl2_ctx* c, int which, double* out, double* r2, const double* in,
                                    const double* active, int nrhs);
