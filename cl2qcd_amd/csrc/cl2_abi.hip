@@ -279,14 +279,19 @@ int run_dslash(cl2_ctx* c, void* out, const void* in, const void* x, const void*
         a.rb  = 1;
         a.lds = 1;
     }
-    if (nrhs > 1 && a.lds && a.rb <= 1) a.map = work_map(c, mrhs_sites_per_block(nrhs, a.lds), 1, t);
+    auto mrhs_map = [&](int staged) {
+        const int sites = mrhs_sites_per_block(nrhs, staged);
+        return fmt == CL2_GAUGE_F16_12 ? work_map(c, sites, 1, t)
+                                       : work_map_mrhs(c, sites, fmt == CL2_GAUGE_F32_12 ? 4 : 8, 24u * nrhs, t);
+    };
+    if (nrhs > 1 && a.lds && a.rb <= 1) a.map = mrhs_map(a.lds);
     CL2_REQUIRE(c, cg_r == nullptr || (cg_alpha != nullptr && norm_res != nullptr), "CG update without its scalars");
     // per-right-hand-side norms come from the kernel with per-site staging (one right-hand side per thread)
     const bool mrhs_norms = nrhs > 1 && norm_res != nullptr;
     if (mrhs_norms) {
         a.rb  = 1;
         a.lds = (lds == 2 && fmt != CL2_GAUGE_F16_12) ? 2 : 1;
-        a.map = work_map(c, mrhs_sites_per_block(nrhs, a.lds), 1, t);
+        a.map = mrhs_map(a.lds);
     }
     CL2_HIP(c, launch_dslash(c, a, fmt));
     // every single-field variant launches blocks_for(Veo, block) blocks, each writing one partial: |out|^2 as a

@@ -271,7 +271,10 @@ __device__ __forceinline__ uint32_t logical_site(const WorkMap& m, uint32_t l)
     const uint32_t zc = l / m.col;
     const uint32_t r  = l - zc * m.col;
     const uint32_t t  = r / m.P;
-    return t * m.half_vs + zc * m.P + (r - t * m.P);
+    const uint32_t q  = r - t * m.P;
+    if (m.row == 0) return t * m.half_vs + zc * m.P + q;
+    const uint32_t z = q / m.row, c = zc / m.ychunks;
+    return t * m.half_vs + (c * (m.P / m.row) + z) * m.plane + (zc - c * m.ychunks) * m.row + (q - z * m.row);
 }
 
 /* logical block of hardware block h under the XCD remap */

@@ -75,6 +75,9 @@ inline unsigned blocks_for(size_t n, int block)
 cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs);
 /* work order of the hopping kernels for this context's lattice and a launch shape */
 WorkMap work_map(const cl2_ctx* c, int block, int nrhs, const cl2_hop_tuning& t);
+/* reals per site from which work_map_mrhs splits slabs in y: 4 Wilson or 12 staggered right-hand sides */
+constexpr uint32_t MRHS_SLAB_REALS = 72;
+WorkMap work_map_mrhs(const cl2_ctx* c, int sites, int real_bytes, uint32_t reals, const cl2_hop_tuning& t);
 /* tuning-table key of the staggered hopping kernel: its link format | DKS_TUNING_KEY */
 constexpr int DKS_TUNING_KEY = 0x100;
 /* sites per block of the multi-RHS kernel that stages links in LDS (blocks of sites x nrhs threads) */

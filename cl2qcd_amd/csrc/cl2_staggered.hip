@@ -474,14 +474,14 @@ hipError_t launch_dks_mrhs(cl2_ctx* c, void* out, const void* in, const void* ga
             if (pairs) {
                 constexpr int SB = DksPair<N>::SB;
                 const unsigned nb = (c->g.veo + SB - 1) / SB;
-                a.map             = work_map(c, SB, 1, t);
+                a.map             = work_map_mrhs(c, SB, 4, 6 * N, t);
                 if (nblocks) *nblocks = nb;
                 hipLaunchKernelGGL((k_dks_eo_mrhs_pair<N>), dim3(nb), dim3(DksPair<N>::BLOCK), 0, c->stream, a);
                 return hipGetLastError();
             }
         }
         constexpr int SB = DksMrhs<N>::SB;
-        a.map = work_map(c, SB, 1, t);
+        a.map = work_map_mrhs(c, SB, F == GAUGE_F32_12 ? 4 : 8, 6 * N, t);
         if (nblocks) *nblocks = (c->g.veo + SB - 1) / SB;
         hipLaunchKernelGGL((k_dks_eo_mrhs<F, N>), dim3((c->g.veo + SB - 1) / SB), dim3(DksMrhs<N>::BLOCK), 0, c->stream,
                            a);

@@ -57,12 +57,16 @@ __host__ __device__ inline size_t link_h8_offset(uint32_t dp, uint32_t eo, uint3
  * a slab is zplanes consecutive z-planes of one t-slice (P = zplanes*ns^2/2 eo
  * sites).  Each of the 8 XCDs gets a contiguous range of logical blocks, so one
  * XCD sweeps its z-chunk through all t and the t+-1 / z+-1 neighbours of a site
- * are still in that XCD's L2. */
+ * are still in that XCD's L2.  With row set a slab holds part of y as well, rows
+ * of y fastest, then z; the slabs of a z-chunk follow each other in y. */
 struct WorkMap {
     uint32_t P;        // eo sites per slab (0: identity order)
     uint32_t col;      // P * nt
     uint32_t half_vs;  // eo sites per t-slice
     uint32_t xcd_q;    // logical blocks per XCD (0: no XCD remap)
+    uint32_t row;      // eo sites of one z-plane in a slab that holds part of y (0: whole planes)
+    uint32_t ychunks;  // slabs of a z-plane in y (row != 0)
+    uint32_t plane;    // eo sites of a z-plane (row != 0)
 };
 
 /* Epilogues fused into the Wilson hopping kernel. */

@@ -15,6 +15,7 @@
 // load their links and full neighbour spinors before either is applied, with
 // a register budget of up to 256 VGPRs, and results leave by streaming
 // stores so they do not evict neighbour spinors from the L2.
+#include <algorithm>
 #include <type_traits>
 
 #include "cl2_device.hpp"
@@ -748,7 +749,7 @@ cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs)
 
 WorkMap work_map(const cl2_ctx* c, int block, int nrhs, const cl2_hop_tuning& t)
 {
-    WorkMap m{0u, 0u, c->g.vs / 2, 0u};
+    WorkMap m{0u, 0u, c->g.vs / 2, 0u, 0u, 0u, 0u};
     const uint32_t ns = c->g.ns, plane = ns * ns / 2;
     int zp            = t.zplanes;
     if (zp < 0) {
@@ -769,6 +770,41 @@ WorkMap work_map(const cl2_ctx* c, int block, int nrhs, const cl2_hop_tuning& t)
     }
     const uint32_t nblocks = (uint32_t)(((size_t)c->g.veo * nrhs + block - 1) / block);
     if (t.xcd && nblocks >= 64) m.xcd_q = nblocks / 8;
+    return m;
+}
+
+/* The order of the staged multi-RHS kernels (sites: sites per block, real_bytes: 8 or 4, reals: reals per site of
+ * the whole block of fields).  nrhs spinors per site make a slab of whole z-planes too large for the three t-slabs
+ * that an XCD sweeps together to stay in its L2, so where the fields exceed the eight L2s a slab also splits y: z
+ * times y rows with a multiple of eight slabs in a t-slice (every XCD sweeps whole ones), at most 2048 sites and
+ * 1.6 MB (FP64) or 2.4 MB (FP32) of spinors, and least halo, counting a y face twice (slabs longer in y measured
+ * faster than square ones).  Without such a slab, and for few reals per site, where this order is no faster, whole
+ * planes.  Measured, whole planes / this order, us per hopping term:
+ *   FP64 12 right-hand sides 24^3x48 540 / 506, 32^3x32 935 / 829, 36^3x32 1534 / 1261, 48^3x32 3539 / 3000, 20^3x40
+ *   280 / 258; 16 of them 32^3x32 1360 / 1133; 4 of them 32^3x64 772 / 715; FP32 12 of them 20^3x40 120 / 109, 36^3x48
+ *   1007 / 948, 48^3x48 2394 / 2219, 32^3x64 874 / 866; 16 of them 32^3x48 854 / 821; staggered FP32 16 of them
+ *   48^3x12 195 / 181, 32^3x48 229 / 226.  FP32 and FP64 of 2, FP16 and staggered ones of 8 moved by -2 to +3 %. */
+WorkMap work_map_mrhs(const cl2_ctx* c, int sites, int real_bytes, uint32_t reals, const cl2_hop_tuning& t)
+{
+    WorkMap m         = work_map(c, sites, 1, t);
+    const uint32_t ns = c->g.ns, row = ns / 2, site_bytes = reals * real_bytes;
+    if (t.zplanes >= 0 || m.xcd_q == 0 || reals < MRHS_SLAB_REALS || (size_t)c->g.veo * site_bytes <= (32u << 20))
+        return m;
+    const uint32_t most = std::min(2048u, (real_bytes == 8 ? 1600000u : 2400000u) / site_bytes);
+    uint32_t bz = 0, by = 0;
+    for (uint32_t z = 1; z <= ns; ++z)
+        for (uint32_t y = 1; y <= ns; ++y) {
+            if (ns % z || ns % y || (ns / z) * (ns / y) % 8 || z * y * row > most) continue;
+            // 1/z + 2/y < 1/bz + 2/by, ties to the larger y
+            const uint32_t f = (y + 2 * z) * bz * by, g = (by + 2 * bz) * z * y;
+            if (bz == 0 || f < g || (f == g && y > by)) bz = z, by = y;
+        }
+    if (bz == 0) return m;
+    m.P       = bz * by * row;
+    m.col     = m.P * c->g.nt;
+    m.row     = by == ns ? 0 : by * row;
+    m.ychunks = ns / by;
+    m.plane   = ns * row;
     return m;
 }
 

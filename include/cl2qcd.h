@@ -455,7 +455,8 @@ int cl2_cg_beta(cl2_ctx* ctx, double* mbeta, double* r2, const double* norms);
 /* ==== launch tuning (no reference counterpart: the reference picks work sizes in
  *      hardware/device_info.cpp:111-128 and hardware/code/opencl_module.cpp get_work_sizes) ==== */
 /* keys: "hop.zplanes" -- z-planes per slab of the t-fastest traversal of the hopping kernels
- *       (-1 heuristic, 0 lexicographic order, else a divisor of ns);
+ *       (-1 by lattice size and format: small lattices in lexicographic order, large multi-RHS blocks in slabs
+ *       that also split y; 0 lexicographic order, else a divisor of ns);
  *       "hop.xcd" -- 1: give each XCD a contiguous range of blocks, 0: hardware round robin;
  *       "hop.block" -- threads per block of the single-field hopping kernel (128, 256, 512);
  *       "hop.occupancy" -- its register budget: 0 (<= 2 waves per SIMD, the two hops of a direction in

@@ -6,7 +6,9 @@
   last block is not full, and fields that are not 16-byte aligned take the one-per-thread kernel;
 * MdagM_eo equals its two D_KS_eo and the elementwise saxpby bit for bit;
 * the streaming multi-shift update agrees with numpy;
-* stage 2 of the reductions sums every one of many partials once.
+* stage 2 of the reductions sums every one of many partials once;
+* the work order of large multi-RHS fields, slabs that split y, visits every site: site order's bits;
+* cl2_scalar_get returns what the stream wrote, on both sides of the mailbox's size.
 """
 import ctypes
 
@@ -173,3 +175,53 @@ def test_many_partial_sums():
                                   s.at(4), s.at(8), s.at(12))
         # unit links and a constant field: D_KS_eo cancels, so <p, A p> = |p|^2 = 1/2
         assert np.abs(s.get()[4:8:2] - 0.5).max() < 1e-6
+
+
+# fields above 32 MiB: slabs of 3 x 6 rows in z and y, 4 x 8 and 5 x 10, and a lattice that no such slab divides
+@pytest.mark.parametrize("fmt,prec,nrhs,ns,nt", [
+    (abi.GAUGE_F64_18, abi.F64, 12, 12, 18), (abi.GAUGE_F64_12, abi.F64, 16, 16, 6), (abi.GAUGE_F64_18, abi.F64, 4, 20, 12),
+    (abi.GAUGE_F32_12, abi.F32, 12, 12, 36), (abi.GAUGE_F32_12, abi.F32, 16, 20, 6), (abi.GAUGE_F32_12, abi.F32, 8, 18, 16)])
+def test_slabs_in_y_visit_every_site(fmt, prec, nrhs, ns, nt):
+    with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        gf = ctx.gauge(random_su3_field(4 * ns ** 3 * nt, 8), fmt)
+        one = ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SPINOR_EO, prec)
+        src = ctx.spinor(prec).upload(np.random.default_rng(9).standard_normal((ctx.veo, 24)))
+        blk, out, got, ref = ctx.buffer(nrhs * one), ctx.buffer(nrhs * one), ctx.spinor(prec), ctx.spinor(prec)
+        for r in range(nrhs):
+            ctx.block_insert_eo(blk.ptr, src.ptr, prec, nrhs, r)
+        for evenodd in (abi.EVEN, abi.ODD):
+            ctx.dslash_eo(ref.ptr, src.ptr, gf.ptr, fmt, evenodd, KAPPA)
+            for r in (0, nrhs - 1):
+                ctx.block_insert_eo(out.ptr, src.ptr, prec, nrhs, r)  # what no block writes would stay the source
+            ctx.dslash_eo_mrhs(out.ptr, blk.ptr, gf.ptr, fmt, evenodd, KAPPA, nrhs)
+            for r in (0, nrhs - 1):
+                ctx.block_extract_eo(got.ptr, out.ptr, prec, nrhs, r)
+                assert np.array_equal(got.download(), ref.download())
+
+
+@pytest.mark.parametrize("fmt,prec,nrhs,ns,nt", [
+    (abi.GAUGE_F64_12, abi.F64, 12, 20, 16), (abi.GAUGE_F32_12, abi.F32, 16, 24, 14), (abi.GAUGE_F32_12, abi.F32, 12, 20, 30)])
+def test_staggered_slabs_in_y_visit_every_site(fmt, prec, nrhs, ns, nt):
+    with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        gf = ctx.gauge(random_su3_field(4 * ns ** 3 * nt, 3)).converted(fmt)
+        one = ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SU3VEC_EO, prec)
+        src = ctx.su3vec(prec).upload(np.random.default_rng(9).standard_normal((ctx.veo, 6)))
+        blk, out, got, ref = ctx.buffer(nrhs * one), ctx.buffer(nrhs * one), ctx.su3vec(prec), ctx.su3vec(prec)
+        for r in range(nrhs):
+            ctx.block_insert_stagg_eo(blk.ptr, src.ptr, prec, nrhs, r)
+        for evenodd in (abi.EVEN, abi.ODD):
+            ctx.D_KS_eo(ref.ptr, src.ptr, gf.ptr, fmt, evenodd)
+            ctx.D_KS_eo_mrhs(out.ptr, blk.ptr, gf.ptr, fmt, evenodd, nrhs)
+            for r in (0, nrhs - 1):
+                ctx.block_extract_stagg_eo(got.ptr, out.ptr, prec, nrhs, r)
+                assert np.array_equal(got.download(), ref.download())
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 200])
+def test_scalar_get(n):
+    with abi.Context(4, 4) as ctx:
+        values = np.random.default_rng(n).standard_normal(n)
+        s = ctx.scalars(n)
+        for shift in range(3):  # successive reads of the one mailbox
+            s.store(values + shift)
+            assert np.array_equal(s.get(), values + shift)
