@@ -363,7 +363,7 @@ static BlockShape block_shape(cl2_ctx* c, size_t n, int prec, int nrhs, int u, b
     for (const void* p : ptrs) wide = wide && (b.pairs || aligned16(p));
     b.cpc    = wide ? 2 : 1;
     b.ncol   = b.pairs ? nrhs : (nrhs % b.cpc == 0 ? nrhs / b.cpc : 1);
-    b.bt     = 256u - (256u % (unsigned)b.ncol);
+    b.bt     = column_block(b.ncol);
     b.nchunk = n / (size_t)b.cpc;
     size_t nb = (b.nchunk + (size_t)b.bt * u - 1) / ((size_t)b.bt * u);
     const size_t cap = partials ? c->npartials / (size_t)nrhs : ((size_t)1 << 22);

@@ -1062,7 +1062,7 @@ __global__ __launch_bounds__(256) void k_block_slot_h(void* block, const void* s
  * per-right-hand-side partials buffer holds (the grid loops beyond) */
 static void block_shape_h(cl2_ctx* c, uint32_t SN, int nrhs, unsigned& bt, unsigned& nb)
 {
-    bt               = 256u - (256u % (unsigned)nrhs);
+    bt               = column_block(nrhs);
     size_t n         = (SN + bt - 1) / bt;
     const size_t cap = c->npartials / (size_t)nrhs;
     nb               = (unsigned)std::max<size_t>(1, std::min(n, std::min(cap, (size_t)BLAS_MAX_BLOCKS)));
@@ -1086,7 +1086,7 @@ hipError_t launch_block_xp_h(cl2_ctx* c, void* x, void* p, const void* r, int nr
 {
     // no partials: two (site, right-hand side) elements per thread over the full grid
     const uint32_t SN = c->g.veo * (uint32_t)nrhs;
-    const unsigned bt = 256u - (256u % (unsigned)nrhs), nb = (SN + 2 * bt - 1) / (2 * bt);
+    const unsigned bt = column_block(nrhs), nb = (SN + 2 * bt - 1) / (2 * bt);
     hipLaunchKernelGGL(k_block_xp_h<2>, dim3(nb), dim3(bt), 0, c->stream, x, p, r, SN, nrhs, alpha, beta);
     return hipGetLastError();
 }

@@ -75,6 +75,14 @@ inline unsigned blocks_for(size_t n, int block)
 cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs);
 /* work order of the hopping kernels for this context's lattice and a launch shape */
 WorkMap work_map(const cl2_ctx* c, int block, int nrhs, const cl2_hop_tuning& t);
+/* threads per block of the elementwise block kernels, a multiple of the ncol chunk columns so that a thread keeps its
+ * right-hand side, and of the wavefront, so that no block starts inside a 128-byte line: 192 rather than 252 threads
+ * for 12 columns (252 / 192: FP32 x and p update at 32^3x64 1119 / 1027 us) */
+constexpr unsigned column_block(int ncol)
+{
+    return 256 % ncol == 0 ? 256u : 192u;  // 1, 2, 4, 8, 16 or 3, 6, 12 columns
+}
+
 /* reals per site from which work_map_mrhs splits slabs in y: 4 Wilson or 12 staggered right-hand sides */
 constexpr uint32_t MRHS_SLAB_REALS = 72;
 WorkMap work_map_mrhs(const cl2_ctx* c, int sites, int real_bytes, uint32_t reals, const cl2_hop_tuning& t);
