@@ -11,8 +11,8 @@
 // XCD's 4 MB L2: every input site is read by 8 output sites, and the fewer
 // sites an XCD has in flight the more of those reads hit.  The single-field
 // kernel therefore keeps few sites in flight (about 4 waves per CU) and gets
-// its memory parallelism from each thread instead: both hops of a direction
-// load their links and full neighbour spinors before either is applied, with
+// its memory parallelism from each thread instead: two to four hops load
+// their links and full neighbour spinors before the first is applied, with
 // a register budget of up to 256 VGPRs, and results leave by streaming
 // stores so they do not evict neighbour spinors from the L2.
 #include <algorithm>
@@ -67,9 +67,6 @@ __device__ __forceinline__ void apply_hop(Cx<R> (&acc)[12], const vec2<R> (&s)[1
     }
 }
 
-/* forward and backward hop of direction DIR: both links and both neighbour spinors (elements nf, nbk
- * of the spinor field) are loaded before either hop is applied.  The forward link is the output
- * site's own (eo index i, parity P), the backward one the neighbour's (eo index linkbk, parity P^1). */
 /* The eight hops of the shapes with four hops' loads in flight (one wave per SIMD, which may stage in AGPRs, or
  * two for FP32).  The four in-plane neighbours (X and Y directions) are gathered component by component: the rows
  * of a block's sites are each other's y neighbours and every site is the x neighbour of two, so what one gather of
@@ -117,7 +114,7 @@ __device__ __forceinline__ void hop_all(Cx<R> (&acc)[12], const vec2<R>* __restr
     apply_hop<3, false>(acc, szb, zb, Cx<R>{R(w.wb[3][0]), R(w.wb[3][1])});
 }
 
-/* the same two hops one after the other, for the 128-VGPR variants: each loads only its own link and
+/* the two hops of direction DIR one after the other, for the 128-VGPR variants: each loads only its own link and
  * neighbour spinor */
 template<int DIR, int FMT, typename R>
 __device__ __forceinline__ void hop_seq(Cx<R> (&acc)[12], const vec2<R>* __restrict__ in, size_t SS, uint32_t nf,
@@ -140,6 +137,9 @@ __device__ __forceinline__ void hop_seq(Cx<R> (&acc)[12], const vec2<R>* __restr
     }
 }
 
+/* forward and backward hop of direction DIR: both links and both neighbour spinors (elements nf, nbk
+ * of the spinor field) are loaded before either hop is applied.  The forward link is the output
+ * site's own (eo index i, parity P), the backward one the neighbour's (eo index linkbk, parity P^1). */
 template<int DIR, int FMT, typename R>
 __device__ __forceinline__ void hop_pair(Cx<R> (&acc)[12], const vec2<R>* __restrict__ in, size_t SS, uint32_t nf,
                                          uint32_t nbk, const void* gauge, uint32_t S, int P, uint32_t i,
