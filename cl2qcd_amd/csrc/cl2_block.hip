@@ -240,22 +240,24 @@ __global__ __launch_bounds__(BLOCK) void k_block_reduce2(const double2* partials
     if (threadIdx.x == 0) {
         const unsigned r = blockIdx.x;
         double2 v        = s;
-        if constexpr (TAIL) {
-            // (|D p_r|^2, |p_r|^2) -> <p_r, (m^2 + sigma_r - D D) p_r> (D_KS anti-hermitian)
+        // (|D p_r|^2, |p_r|^2) -> <p_r, (m^2 + sigma_r - D D) p_r> (D_KS anti-hermitian)
+        if constexpr (TAIL)
             if (tail.kind == TAIL_ALPHA_MDAGM) v = make_double2(tail.coef[r] * s.y + s.x, 0.);
-            double2 al = make_double2(0., 0.);
-            if (tail.active[r] != 0.)
-                al = tail.kind == TAIL_ALPHA ? block_alpha(tail.r2[r], v.x, v.y)
-                                             : make_double2(tail.r2[r] * v.x / (v.x * v.x), 0.);
-            tail.alpha[2 * r]     = al.x;
-            tail.alpha[2 * r + 1] = al.y;
-        }
         if (out_kind == 0) {
             res[2 * r]     = v.x;
             res[2 * r + 1] = v.y;
         } else {
             res[r] = v.x;
         }
+        if constexpr (TAIL)
+            if (tail.alpha) {
+                double2 al = make_double2(0., 0.);
+                if (tail.active[r] != 0.)
+                    al = tail.kind == TAIL_ALPHA ? block_alpha(tail.r2[r], v.x, v.y)
+                                                 : make_double2(tail.r2[r] * v.x / (v.x * v.x), 0.);
+                tail.alpha[2 * r]     = al.x;
+                tail.alpha[2 * r + 1] = al.y;
+            }
     }
 }
 
@@ -377,6 +379,25 @@ constexpr int BLOCK_U_REDUCE = 4;
 hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, double* res, int out_kind, int nrhs,
                                 const SumTail* tail)
 {
+    // The step lengths are formed by each right-hand side's own block, in any order.  Where a caller's arrays overlap,
+    // one block's alpha or sum could land on what another has yet to read: a launch after all the sums forms them then
+    SumTail sums_only;
+    if (tail && tail->alpha) {
+        auto apart = [](const double* a, int na, const double* b, int nb_) {
+            const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+            return x + na * sizeof(double) <= y || y + nb_ * sizeof(double) <= x;
+        };
+        const int n = nrhs;
+        if (!(apart(tail->alpha, 2 * n, res, 2 * n) && apart(tail->alpha, 2 * n, tail->r2, n) &&
+              apart(tail->alpha, 2 * n, tail->active, n) && apart(res, 2 * n, tail->r2, n) &&
+              apart(res, 2 * n, tail->active, n))) {
+            sums_only       = *tail;
+            sums_only.alpha = nullptr;
+            const hipError_t e = launch_block_reduce2(c, parts, nb, res, out_kind, nrhs, &sums_only);
+            if (e != hipSuccess) return e;
+            return launch_block_cg_scalars(c, 0, tail->alpha, const_cast<double*>(tail->r2), res, tail->active, nrhs);
+        }
+    }
     auto go = [&](auto kernel, auto t) {
         hipLaunchKernelGGL(kernel, dim3(nrhs), dim3(1024), 0, c->stream, parts, nb, res, out_kind, t);
     };

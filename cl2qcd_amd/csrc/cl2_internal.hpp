@@ -151,7 +151,8 @@ unsigned reduce_stage1_blocks(size_t n, int prec, const void* x, const void* y);
 /* scalar work that the block finishing a stage-2 sum does with it, instead of a launch of its own:
  *   TAIL_RATIO       alpha = r2 / sum (complex scalars, as cl2_complex_op's ratio);
  *   TAIL_CGM_BETA    pap = m2 sum.y + sum.x; beta_prev = beta; beta = 0 - r2 / pap (the CG-M step on MdagM_eo);
- *   TAIL_ALPHA       per right-hand side: alpha = r2 / sum where active, else 0 (cl2_block_cg_alpha);
+ *   TAIL_ALPHA       per right-hand side: alpha = r2 / sum where active, else 0 (cl2_block_cg_alpha; without alpha the
+ *                    sum only);
  *   TAIL_ALPHA_MDAGM the same with sum replaced by coef sum.y + sum.x, also left in its place (the lockstep step on
  *                    MdagM_eo + sigma) */
 enum SumTailKind : int { TAIL_RATIO = 1, TAIL_CGM_BETA = 2, TAIL_ALPHA = 3, TAIL_ALPHA_MDAGM = 4 };

@@ -225,3 +225,43 @@ def test_scalar_get(n):
         for shift in range(3):  # successive reads of the one mailbox
             s.store(values + shift)
             assert np.array_equal(s.get(), values + shift)
+
+
+@pytest.mark.parametrize("shared", ["pAp", "r2", "active"])
+@pytest.mark.parametrize("staggered", [False, True])
+def test_lockstep_step_with_shared_arrays(staggered, shared):
+    # the step lengths may take the place of the sums, of the old norms or of the active flags: the residual that
+    # follows has the bits that separate arrays give
+    ns, nt, n, fmt, prec = 6, 10, 8, abi.GAUGE_F64_18, abi.F64
+    with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        gf = ctx.gauge(random_su3_field(4 * 2 * ctx.veo, 3))
+        field = abi.FIELD_SU3VEC_EO if staggered else abi.FIELD_SPINOR_EO
+        one = ctx.lib.cl2_field_bytes(ctx.handle, field, prec)
+        p, tmp = ctx.buffer(n * one), ctx.buffer(2 * n * one)
+        got = []
+        for separate in (True, False):
+            r, f = ctx.buffer(n * one), ctx.su3vec(prec) if staggered else ctx.spinor(prec)
+            insert, extract = ((ctx.block_insert_stagg_eo, ctx.block_extract_stagg_eo) if staggered
+                               else (ctx.block_insert_eo, ctx.block_extract_eo))
+            for k in range(n):
+                ctx.gaussian_eo(field, f.ptr, prec, 10 + k)
+                insert(p.ptr, f.ptr, prec, n, k)
+                ctx.gaussian_eo(field, f.ptr, prec, 50 + k)
+                insert(r.ptr, f.ptr, prec, n, k)
+            s = ctx.scalars(8 * n)
+            r2, active, pap, norms, alpha = s.at(0), s.at(2 * n), s.at(4 * n), s.at(6 * n), ctx.scalars(2 * n)
+            s.store(np.concatenate([np.linspace(0.5, 2.0, 2 * n), np.ones(n - 1), np.zeros(5 * n + 1)]))
+            a = alpha.ptr if separate else {"pAp": pap, "r2": r2, "active": active}[shared]
+            if staggered:
+                ctx.MdagM_eo_mrhs_cg_step(r.ptr, p.ptr, gf.ptr, fmt, 0.1, abi.EVEN, None, tmp.ptr, n, r2, active, pap, a,
+                                          norms)
+            else:
+                ctx.fermionmatrix_eo_mrhs_cg_step(abi.OP_QPLUSQMINUS_EO, r.ptr, p.ptr, gf.ptr, fmt,
+                                                  abi.ACTION_TWISTEDMASS, KAPPA, MUBAR, None, None, tmp.ptr, n, r2,
+                                                  active, pap, a, norms)
+            fields = []
+            for k in range(n):
+                extract(f.ptr, r.ptr, prec, n, k)
+                fields.append(f.download())
+            got.append((np.stack(fields), s.get()[6 * n:]))
+        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
