@@ -5,7 +5,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -470,13 +469,13 @@ int cl2_ctx_create(cl2_ctx** out, int device, const cl2_lattice* lat)
         hipMalloc(&c->partials, c->npartials * 2 * sizeof(double)) != hipSuccess ||
         hipMalloc(&c->dscratch, 64 * sizeof(double)) != hipSuccess ||
         hipMalloc(&c->ptr_table, 128 * sizeof(void*)) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&c->mail), sizeof(cl2_mailbox), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&c->mail.box), sizeof(cl2_mailbox), hipHostMallocDefault) != hipSuccess ||
         hipEventCreate(&c->ev_start) != hipSuccess || hipEventCreate(&c->ev_stop) != hipSuccess) {
         cl2_ctx_destroy(c);
         return create_fail(CL2_E_HIP, "context allocation failed");
     }
-    c->mail->number = 0;
-    *out            = c;
+    c->mail.box->number = 0;
+    *out                = c;
     return CL2_OK;
 }
 
@@ -488,7 +487,7 @@ int cl2_ctx_destroy(cl2_ctx* c)
     if (c->partials) (void)hipFree(c->partials);
     if (c->dscratch) (void)hipFree(c->dscratch);
     if (c->ptr_table) (void)hipFree(c->ptr_table);
-    if (c->mail) (void)hipHostFree(c->mail);
+    if (c->mail.box) (void)hipHostFree(c->mail.box);
     if (c->ev_start) (void)hipEventDestroy(c->ev_start);
     if (c->ev_stop) (void)hipEventDestroy(c->ev_stop);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -843,16 +842,9 @@ int cl2_scalar_get(cl2_ctx* c, double* host, const double* dev, int n)
     // enqueued so far, and the host watches the transfer's number for a while before it waits on the stream (which
     // also reports what went wrong where the number never comes).  A copy to pageable memory and a wait on the stream
     // cost about 15 us more per read: FP16-inner CG on 16^3x32, one read per iteration, 30.7 against 25.5 ms
-    std::lock_guard<std::mutex> lk(c->mail_mutex);
-    const uint64_t number = __atomic_load_n(&c->mail->number, __ATOMIC_RELAXED) + 1;
-    CL2_HIP(c, launch_mail(c, dev, n, number));
-    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
-    while (__atomic_load_n(&c->mail->number, __ATOMIC_ACQUIRE) != number)
-        if (std::chrono::steady_clock::now() > until) {
-            CL2_HIP(c, hipStreamSynchronize(c->stream));
-            break;
-        }
-    std::memcpy(host, c->mail->value, n * sizeof(double));
+    CL2_HIP(c, c->mail.read(
+                   host, n, [&](uint64_t number) { return launch_mail(c, dev, n, number); },
+                   [&] { return hipStreamSynchronize(c->stream); }));
     return CL2_OK;
 }
 

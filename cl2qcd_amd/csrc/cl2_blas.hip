@@ -518,7 +518,7 @@ __global__ __launch_bounds__(cl2_mailbox::SIZE) void k_mail(cl2_mailbox* m, cons
 
 hipError_t launch_mail(cl2_ctx* c, const double* src, int n, uint64_t number)
 {
-    hipLaunchKernelGGL(k_mail, dim3(1), dim3(cl2_mailbox::SIZE), 0, c->stream, c->mail, src, n, number);
+    hipLaunchKernelGGL(k_mail, dim3(1), dim3(cl2_mailbox::SIZE), 0, c->stream, c->mail.box, src, n, number);
     return hipGetLastError();
 }
 

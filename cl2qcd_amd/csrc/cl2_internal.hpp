@@ -4,11 +4,11 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
-#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
 
+#include "cl2_mailbox.hpp"
 #include "cl2_types.hpp"
 
 /* launch shape of the hopping kernels */
@@ -22,13 +22,6 @@ struct cl2_hop_tuning {
                   // four hops in flight), 4 (>= 4 waves, one hop at a time); -1: the format's default
 };
 
-/* scalars on their way to the host: the values, then the number of the transfer they belong to */
-struct cl2_mailbox {
-    static constexpr int SIZE = 64;
-    double value[SIZE];
-    uint64_t number;
-};
-
 struct cl2_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -39,8 +32,7 @@ struct cl2_ctx {
     double* partials = nullptr;  // reduction scratch: one double2 per block
     size_t npartials = 0;
     double* dscratch = nullptr;  // a few device doubles for host-read results
-    cl2_mailbox* mail = nullptr; // pinned host memory that a kernel writes scalars into (cl2_scalar_get)
-    std::mutex mail_mutex;       // one reader of the mailbox at a time
+    cl2_mail_reader mail;        // pinned host memory that a kernel writes scalars into (cl2_scalar_get)
     void** ptr_table = nullptr;  // device copy of the field-pointer table of the multi-shift update (2 x 64)
     std::vector<void*> ptr_table_host;  // what ptr_table holds
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
