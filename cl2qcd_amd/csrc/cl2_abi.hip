@@ -829,11 +829,31 @@ int cl2_scalar_store(cl2_ctx* c, double* dev, const double* host, int n)
     return CL2_OK;
 }
 
+/* whether a kernel on the context's stream may read these bytes now: memory of the context's own device, to its end,
+ * and no capture that would record the kernel.  A copy refuses or serves the rest (host memory, another device's, a
+ * range that leaves its allocation); a kernel would fault on it. */
+static bool readable_by_kernel(cl2_ctx* c, const void* p, size_t bytes)
+{
+    hipPointerAttribute_t at{};
+    hipDeviceptr_t base = nullptr;
+    size_t size         = 0;
+    hipStreamCaptureStatus capture;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess ||
+        hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess ||
+        hipStreamIsCapturing(c->stream, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const size_t offset = (size_t)(static_cast<const char*>(p) - static_cast<const char*>(base));
+    return at.type == hipMemoryTypeDevice && at.device == c->device && offset <= size && bytes <= size - offset &&
+           capture == hipStreamCaptureStatusNone;
+}
+
 int cl2_scalar_get(cl2_ctx* c, double* host, const double* dev, int n)
 {
     if (!c) return CL2_E_ARG;
     CL2_REQUIRE(c, dev && host && n > 0, "bad scalar get");
-    if (n > cl2_mailbox::SIZE) {
+    if (n > cl2_mailbox::SIZE || !readable_by_kernel(c, dev, n * sizeof(double))) {
         CL2_HIP(c, hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         CL2_HIP(c, hipStreamSynchronize(c->stream));
         return CL2_OK;

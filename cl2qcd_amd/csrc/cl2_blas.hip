@@ -518,8 +518,9 @@ __global__ __launch_bounds__(cl2_mailbox::SIZE) void k_mail(cl2_mailbox* m, cons
 
 hipError_t launch_mail(cl2_ctx* c, const double* src, int n, uint64_t number)
 {
-    hipLaunchKernelGGL(k_mail, dim3(1), dim3(cl2_mailbox::SIZE), 0, c->stream, c->mail.box, src, n, number);
-    return hipGetLastError();
+    // the launch's own result: an error that an earlier call left behind is no reason to refuse a read
+    void* args[] = {&c->mail.box, &src, &n, &number};
+    return hipLaunchKernel(reinterpret_cast<const void*>(k_mail), dim3(1), dim3(cl2_mailbox::SIZE), args, 0, c->stream);
 }
 
 hipError_t launch_vec_element(cl2_ctx* c, double* out, const double* in, int out_index, int in_index)

@@ -265,3 +265,14 @@ def test_lockstep_step_with_shared_arrays(staggered, shared):
                 fields.append(f.download())
             got.append((np.stack(fields), s.get()[6 * n:]))
         assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+def test_scalar_get_refuses_what_a_copy_refuses():
+    # a range beyond its allocation, and host memory: errors, and the next read is the scalar's again
+    with abi.Context(4, 4) as ctx:
+        s = ctx.scalars(4)
+        s.store([1.0, 2.0, 3.0, 4.0])
+        out, host = np.zeros(64), np.arange(64.0)
+        for src, n in ((s.ptr, 64), (s.at(3), 2), (host.ctypes.data, 2)):
+            assert ctx.lib.cl2_scalar_get(ctx.handle, out.ctypes.data, src, n) != 0
+            assert np.array_equal(s.get(), [1.0, 2.0, 3.0, 4.0])
