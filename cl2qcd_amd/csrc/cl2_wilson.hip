@@ -73,10 +73,13 @@ __device__ __forceinline__ void apply_hop(Cx<R> (&acc)[12], const vec2<R> (&s)[1
  * a component brings into the 32 KiB L1 (4 KiB for 256 sites and one 16-byte component) the next ones find there.
  * Gathering spinor by spinor (two directions at a time, four spinors of 48 KiB each per block) found none of it:
  * the L1 asked the L2 for every gathered byte, 112 M lines per launch at 48^3x96 in FP64.  Measured, spinor by
- * spinor / component by component, one run: F64_18 1516 / 1481 us at 48^3x96, 98.9 / 94.3 us at 24^3x48, 289 /
- * 279 us at 32^3x64; F64_12 1147 / 1143 us and F32 555 / 545 us at 48^3x96.  The hops are applied in the order
- * T, X, Y, Z (the X and Y links are loaded once the T hops have freed their registers, the Z hops' data once the X
- * hops have), so every variant computes the same bits. */
+ * spinor / component by component, us per hopping term on one stream (three contexts at once in brackets): F64_18
+ * 1518 / 1482 (1625 / 1612) at 48^3x96, 292 / 286 (303 / 301) at 32^3x64, 99.2 / 94.5 (96.1 / 94.4) at 24^3x48; F32
+ * 558 / 546 (591 / 584) at 48^3x96.  F64_12 stays spinor by spinor (hop_quad): 1151 / 1162 (1220 / 1246) at 48^3x96,
+ * 230 / 221 (230 / 235) at 32^3x64, 78.8 / 76.5 (70.7 / 72.8) at 24^3x48, 14.5 / 15.1 (14.2 / 14.1) at 16^3x32, 13.6 /
+ * 14.9 (11.8 / 11.9) at 14^3x40: gathering by component is ahead only alone on the device and from 24^3x30 to
+ * 32^3x64.  The hops are applied in the order T, X, Y, Z (the X and Y links are loaded once the T hops have freed
+ * their registers, the Z hops' data once the X hops have), so every variant computes the same bits. */
 template<int FMT, int NRHS, typename R>
 __device__ __forceinline__ void hop_all(Cx<R> (&acc)[12], const vec2<R>* __restrict__ in, size_t SS, const SiteNb& nb,
                                         uint32_t rhs, const void* gauge, uint32_t S, int P, uint32_t i,
@@ -112,6 +115,29 @@ __device__ __forceinline__ void hop_all(Cx<R> (&acc)[12], const vec2<R>* __restr
     apply_hop<2, false>(acc, sp[3], yb, Cx<R>{R(w.wb[2][0]), R(w.wb[2][1])});
     apply_hop<3, true>(acc, szf, zf, Cx<R>{R(w.wf[3][0]), R(w.wf[3][1])});
     apply_hop<3, false>(acc, szb, zb, Cx<R>{R(w.wb[3][0]), R(w.wb[3][1])});
+}
+
+/* The same loads two directions at a time: four links and four whole neighbour spinors in flight before any hop is
+ * applied. */
+template<int D0, int D1, int FMT, int NRHS, typename R>
+__device__ __forceinline__ void hop_quad(Cx<R> (&acc)[12], const vec2<R>* __restrict__ in, size_t SS, const SiteNb& nb,
+                                         uint32_t rhs, const void* gauge, uint32_t S, int P, uint32_t i,
+                                         const HopWeights<double>& w)
+{
+    Su3<R> u0f, u0b, u1f, u1b;
+    vec2<R> s0f[12], s0b[12], s1f[12], s1b[12];
+    GaugeLoad<FMT>::load(gauge, S, D0, P, i, u0f);
+    GaugeLoad<FMT>::load(gauge, S, D0, P ^ 1, nb.dn[D0], u0b);
+    GaugeLoad<FMT>::load(gauge, S, D1, P, i, u1f);
+    GaugeLoad<FMT>::load(gauge, S, D1, P ^ 1, nb.dn[D1], u1b);
+    load_spinor<R>(s0f, in, SS, (size_t)nb.up[D0] * NRHS + rhs);
+    load_spinor<R>(s0b, in, SS, (size_t)nb.dn[D0] * NRHS + rhs);
+    load_spinor<R>(s1f, in, SS, (size_t)nb.up[D1] * NRHS + rhs);
+    load_spinor<R>(s1b, in, SS, (size_t)nb.dn[D1] * NRHS + rhs);
+    apply_hop<D0, true>(acc, s0f, u0f, Cx<R>{R(w.wf[D0][0]), R(w.wf[D0][1])});
+    apply_hop<D0, false>(acc, s0b, u0b, Cx<R>{R(w.wb[D0][0]), R(w.wb[D0][1])});
+    apply_hop<D1, true>(acc, s1f, u1f, Cx<R>{R(w.wf[D1][0]), R(w.wf[D1][1])});
+    apply_hop<D1, false>(acc, s1b, u1b, Cx<R>{R(w.wb[D1][0]), R(w.wb[D1][1])});
 }
 
 /* the two hops of direction DIR one after the other, for the 128-VGPR variants: each loads only its own link and
@@ -214,13 +240,14 @@ __device__ __forceinline__ void hop_pair(Cx<R> (&acc)[12], const vec2<R>* __rest
  *   OCC = 0: at most 2 waves per SIMD (up to 256 VGPRs), the two hops of one direction in flight;
  *   OCC = 1: 1 wave per SIMD, four hops and more in flight (hop_all; blocks of at most 256);
  *   OCC = 2: the same at at most 2 waves per SIMD (FP32);
+ *   OCC = 3: 1 wave per SIMD, the four hops of two directions in flight (hop_quad);
  *   OCC = 4: at least 4 waves per SIMD (at most 128 VGPRs), one hop at a time.
  * PLAIN: the plain hopping term (no epilogue, no norms), compiled without the epilogue's branches and the
  * block reduction; same arithmetic (a standalone copy measured 0.8 % faster than the general kernel for FP64
  * 18-real links at 48^3x96 in one run, within the spread between boxes in the benchmark). */
 template<int FMT, int BLOCK, int NRHS, int OCC = 0, bool PLAIN = false>
 __global__ __launch_bounds__(BLOCK)
-__attribute__((amdgpu_waves_per_eu(OCC == 4 ? 4 : 1, OCC == 4 ? 8 : (OCC == 1 ? 1 : 2))))
+__attribute__((amdgpu_waves_per_eu(OCC == 4 ? 4 : 1, OCC == 4 ? 8 : (OCC == 1 || OCC == 3 ? 1 : 2))))
 void k_dslash_eo(typename std::conditional<NRHS == 1, DslashArgs, DslashRhsArgs>::type a)
 {
     using R = typename GaugeLoad<FMT>::R;
@@ -249,6 +276,9 @@ void k_dslash_eo(typename std::conditional<NRHS == 1, DslashArgs, DslashRhsArgs>
                          CL2_W(wf, m), CL2_W(wb, m));
         if constexpr (OCC == 1 || OCC == 2) {
             hop_all<FMT, NRHS>(acc, in, SS, nb, rhs, a.gauge, S, P, i, a.w);
+        } else if constexpr (OCC == 3) {
+            hop_quad<0, 1, FMT, NRHS>(acc, in, SS, nb, rhs, a.gauge, S, P, i, a.w);
+            hop_quad<2, 3, FMT, NRHS>(acc, in, SS, nb, rhs, a.gauge, S, P, i, a.w);
         } else {
             CL2_DIR(0)
             CL2_DIR(1)
@@ -906,15 +936,16 @@ static hipError_t launch_dslash_n(cl2_ctx* c, const DslashRhsArgs& ra, int forma
             // the 1-wave-per-SIMD shapes (blocks of 128 or 256), the 128-VGPR shapes and the four-hops-in-
             // 256-VGPRs shapes for FP32 only (the FP64 kernels spill at those budgets)
             const bool plain = a.epilogue == EPI_PLAIN && !a.norm_partials && !a.cg_r && !a.per_rhs && !a.gamma5;
+            constexpr int ONE_WAVE = F == GAUGE_F64_12 ? 3 : 1;  // hop_all's comment has the figures
             if (a.occ == 1 && bs == 128) {
-                hipLaunchKernelGGL((k_dslash_eo<F, 128, 1, 1>), dim3(nb), dim3(128), 0, c->stream, a);
+                hipLaunchKernelGGL((k_dslash_eo<F, 128, 1, ONE_WAVE>), dim3(nb), dim3(128), 0, c->stream, a);
                 return hipGetLastError();
             }
             if (a.occ == 1 && bs != 512) {
                 if (plain)
-                    hipLaunchKernelGGL((k_dslash_eo<F, 256, 1, 1, true>), dim3(nb), dim3(256), 0, c->stream, a);
+                    hipLaunchKernelGGL((k_dslash_eo<F, 256, 1, ONE_WAVE, true>), dim3(nb), dim3(256), 0, c->stream, a);
                 else
-                    hipLaunchKernelGGL((k_dslash_eo<F, 256, 1, 1>), dim3(nb), dim3(256), 0, c->stream, a);
+                    hipLaunchKernelGGL((k_dslash_eo<F, 256, 1, ONE_WAVE>), dim3(nb), dim3(256), 0, c->stream, a);
                 return hipGetLastError();
             }
             if constexpr (F == GAUGE_F32_12) {

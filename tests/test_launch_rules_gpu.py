@@ -276,3 +276,27 @@ def test_scalar_get_refuses_what_a_copy_refuses():
         for src, n in ((s.ptr, 64), (s.at(3), 2), (host.ctypes.data, 2)):
             assert ctx.lib.cl2_scalar_get(ctx.handle, out.ctypes.data, src, n) != 0
             assert np.array_equal(s.get(), [1.0, 2.0, 3.0, 4.0])
+
+
+@pytest.mark.parametrize("block", [128, 256])
+@pytest.mark.parametrize("ns,nt", [(6, 10), (12, 28)])  # a last block of 56 sites; with the XCD remap
+def test_f64_12_gather_order_keeps_the_bits(ns, nt, block):
+    # 12-real FP64 links gather two directions at a time where a wave has a SIMD to itself: the bits of the shape with
+    # two hops in flight, plain and with the epilogue
+    with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        gf = ctx.gauge(seed=3, epsilon=0.35).converted(abi.GAUGE_F64_12)
+        a, b = ctx.spinor(), ctx.spinor()
+        tmp = ctx.buffer(2 * ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SPINOR_EO, abi.F64))
+        ctx.gaussian_eo(abi.FIELD_SPINOR_EO, a.ptr, abi.F64, 5)
+        ctx.tune_set(b"hop.block", block)
+        got = []
+        for occ in (1, 0):
+            ctx.tune_set(b"hop.occupancy", occ)
+            for evenodd in (abi.EVEN, abi.ODD):
+                ctx.dslash_eo(b.ptr, a.ptr, gf.ptr, abi.GAUGE_F64_12, evenodd, KAPPA)
+                got.append(b.download())
+            ctx.fermionmatrix_eo(abi.OP_AEE_MINUS_AND_GAMMA5, b.ptr, a.ptr, gf.ptr, abi.GAUGE_F64_12,
+                                 abi.ACTION_TWISTEDMASS, KAPPA, MUBAR, tmp.ptr)
+            got.append(b.download())
+        for x, y in zip(got[:3], got[3:]):
+            assert np.array_equal(x, y)
