@@ -56,10 +56,14 @@ int fail(cl2_ctx* c, int code, const std::string& msg)
     return code;
 }
 
+/* the error is the caller's from here on: the runtime's own note of it would fail the thread's next launch as well */
 #define CL2_HIP(ctx, call)                                                                         \
     do {                                                                                           \
         hipError_t e_ = (call);                                                                    \
-        if (e_ != hipSuccess) return fail(ctx, CL2_E_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
+        if (e_ != hipSuccess) {                                                                    \
+            (void)hipGetLastError();                                                               \
+            return fail(ctx, CL2_E_HIP, std::string(#call) + ": " + hipGetErrorString(e_));        \
+        }                                                                                          \
     } while (0)
 
 #define CL2_REQUIRE(ctx, cond, msg) \

@@ -268,7 +268,7 @@ def test_lockstep_step_with_shared_arrays(staggered, shared):
 
 
 def test_scalar_get_refuses_what_a_copy_refuses():
-    # a range beyond its allocation, and host memory: errors, and the next read is the scalar's again
+    # a range beyond its allocation, and host memory: errors, and the next read and the next launch are in order again
     with abi.Context(4, 4) as ctx:
         s = ctx.scalars(4)
         s.store([1.0, 2.0, 3.0, 4.0])
@@ -276,6 +276,8 @@ def test_scalar_get_refuses_what_a_copy_refuses():
         for src, n in ((s.ptr, 64), (s.at(3), 2), (host.ctypes.data, 2)):
             assert ctx.lib.cl2_scalar_get(ctx.handle, out.ctypes.data, src, n) != 0
             assert np.array_equal(s.get(), [1.0, 2.0, 3.0, 4.0])
+            ctx.scalar_copy(s.at(1), s.at(1) + 8, 1)
+            s.store([1.0, 2.0, 3.0, 4.0])
 
 
 @pytest.mark.parametrize("block", [128, 256])
