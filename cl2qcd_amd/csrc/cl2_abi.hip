@@ -1817,24 +1817,20 @@ int cl2_tune_set(cl2_ctx* c, const char* key, long value)
         CL2_REQUIRE(c, value == -1 || value == 0 || (value > 0 && c->g.ns % (uint32_t)value == 0),
                     "hop.zplanes must be -1, 0 or a divisor of ns");
         c->tune_zplanes = (int)value;
-        c->tune_manual  = true;
         return CL2_OK;
     }
     if (k == "hop.xcd") {
-        c->tune_xcd    = value ? 1 : 0;
-        c->tune_manual = true;
+        c->tune_xcd = value ? 1 : 0;
         return CL2_OK;
     }
     if (k == "mrhs.rb") {
         CL2_REQUIRE(c, value == 0 || value == 1 || value == 2 || value == 4, "mrhs.rb must be 0, 1, 2 or 4");
         c->tune_mrhs_rb = (int)value;
-        c->tune_manual  = true;
         return CL2_OK;
     }
     if (k == "mrhs.lds") {
         CL2_REQUIRE(c, value == 0 || value == 1 || value == 2, "mrhs.lds must be 0, 1 or 2");
         c->tune_mrhs_lds = (int)value;
-        c->tune_manual   = true;
         return CL2_OK;
     }
     if (k == "mrhs.off32") {
@@ -1842,16 +1838,15 @@ int cl2_tune_set(cl2_ctx* c, const char* key, long value)
         return CL2_OK;
     }
     if (k == "hop.block") {
-        CL2_REQUIRE(c, value == 128 || value == 256 || value == 512, "hop.block must be 128, 256 or 512");
-        c->tune_block  = (int)value;
-        c->tune_manual = true;
+        CL2_REQUIRE(c, value == 0 || value == SPLIT_SITES || value == 128 || value == 256 || value == 512,
+                    "hop.block must be 0, 64, 128, 256 or 512");
+        c->tune_block = (int)value;
         return CL2_OK;
     }
     if (k == "hop.occupancy") {
         CL2_REQUIRE(c, value == -1 || value == 0 || value == 1 || value == 2 || value == 4,
                     "hop.occupancy must be -1, 0, 1, 2 or 4");
-        c->tune_occ    = (int)value;
-        c->tune_manual = true;
+        c->tune_occ = (int)value;
         return CL2_OK;
     }
     return fail(c, CL2_E_ARG, "unknown tuning key " + k);
@@ -1862,14 +1857,41 @@ long cl2_tune_get(const cl2_ctx* c, const char* key)
     if (!c || !key) return -2;
     const std::string k(key);
     if (k == "hop.zplanes") return c->tune_zplanes;
-    if (k == "hop.xcd") return c->tune_xcd;
+    if (k == "hop.xcd") return c->tune_xcd != 0;
     if (k == "mrhs.rb") return c->tune_mrhs_rb;
     if (k == "hop.block") return c->tune_block;
-    if (k == "mrhs.lds") return c->tune_mrhs_lds;
+    if (k == "mrhs.lds") return c->tune_mrhs_lds >= 0 ? c->tune_mrhs_lds : 1;
     if (k == "mrhs.off32") return c->tune_mrhs_off32;
     if (k == "hop.occupancy") return c->tune_occ;
+    const char* formats[] = {"f64_18", "f64_12", "f32_12", "f16_12"};
+    const int numbers[]   = {CL2_GAUGE_F64_18, CL2_GAUGE_F64_12, CL2_GAUGE_F32_12, CL2_GAUGE_F16_12};
+    for (int f = 0; f < 4; ++f)
+        if (k == std::string("hop.block.") + formats[f]) return hop_tuning(c, numbers[f], 1).block;
     return -2;
 }
+
+/* puts what is set by hand aside while the autotuner times its own shapes */
+struct HandSettings {
+    cl2_ctx* c;
+    int zplanes, xcd, rb, lds, block, occ;
+    explicit HandSettings(cl2_ctx* ctx)
+        : c(ctx), zplanes(ctx->tune_zplanes), xcd(ctx->tune_xcd), rb(ctx->tune_mrhs_rb), lds(ctx->tune_mrhs_lds),
+          block(ctx->tune_block), occ(ctx->tune_occ)
+    {
+        c->tune_zplanes = c->tune_xcd = c->tune_mrhs_lds = c->tune_occ = -1;
+        c->tune_mrhs_rb = c->tune_block = 0;
+    }
+    HandSettings(const HandSettings&) = delete;
+    ~HandSettings()
+    {
+        c->tune_zplanes  = zplanes;
+        c->tune_xcd      = xcd;
+        c->tune_mrhs_rb  = rb;
+        c->tune_mrhs_lds = lds;
+        c->tune_block    = block;
+        c->tune_occ      = occ;
+    }
+};
 
 /* Autotuner of the hopping kernel's launch shape: every candidate (z-planes per slab, XCD mapping,
  * right-hand sides per thread) is timed with HIP events on scratch fields and the caller's gauge field;
@@ -1903,15 +1925,15 @@ int cl2_autotune_dslash(cl2_ctx* c, const void* gauge, int fmt, int nrhs, double
     if (nrhs > 1)
         for (int r : {2, 4})
             if (nrhs % r == 0) rbs.push_back(r);
-    // (block, occupancy hint) shapes of the single-field kernel
+    // (sites per block, occupancy hint) shapes of the single-field kernel: the wave-per-hop kernel among them
     std::vector<std::pair<int, int>> shapes = {{256, 0}};
     if (nrhs == 1 && fmt == CL2_GAUGE_F32_12)
         shapes = {{256, 0}, {128, 0}, {512, 0}, {256, 1}, {128, 1}, {256, 2}, {128, 2}, {256, 4}, {128, 4}};
     else if (nrhs == 1 && fmt == CL2_GAUGE_F16_12)
         shapes = {{256, 0}, {128, 0}, {512, 0}, {256, 1}, {128, 1}, {256, 4}, {128, 4}};
     else if (nrhs == 1) shapes = {{256, 0}, {128, 0}, {512, 0}, {256, 1}, {128, 1}};
-    const bool manual = c->tune_manual;
-    c->tune_manual    = false;
+    if (nrhs == 1) shapes.push_back({SPLIT_SITES, 0});
+    const HandSettings unset(c);
     const double one[2] = {1., 0.};
     double best         = 1e30;
     cl2_hop_tuning bt{-1, 1, 1, 1, DSLASH_BLOCK, -1};
@@ -1969,7 +1991,6 @@ int cl2_autotune_dslash(cl2_ctx* c, const void* gauge, int fmt, int nrhs, double
             }
         }
     }
-    c->tune_manual = manual;
     if (rc) {
         c->tuned.erase({fmt, nrhs});
         return rc;
@@ -1979,7 +2000,7 @@ int cl2_autotune_dslash(cl2_ctx* c, const void* gauge, int fmt, int nrhs, double
     if (zplanes) *zplanes = bt.zplanes;
     if (xcd) *xcd = bt.xcd;
     if (rb) *rb = (nrhs > 1 && bt.rb <= 1 && bt.lds) ? -bt.lds : bt.rb;
-    if (block) *block = bt.block;
+    if (block) *block = bt.block == SPLIT_SITES ? SPLIT_BLOCK : bt.block;
     if (occupancy) *occupancy = bt.occ;
     return CL2_OK;
 }
@@ -2003,9 +2024,8 @@ int cl2_autotune_dks(cl2_ctx* c, const void* gauge, int fmt, double* best_ms, in
     const std::vector<std::pair<int, int>> shapes = {{256, 0}, {128, 0}, {512, 0}, {256, 1}, {128, 1}, {256, 4},
                                                      {128, 4}};
     const std::pair<int, int> key{fmt | DKS_TUNING_KEY, 1};
-    const bool manual = c->tune_manual;
-    c->tune_manual    = false;
-    double best       = 1e30;
+    const HandSettings unset(c);
+    double best = 1e30;
     cl2_hop_tuning bt{-1, 1, 1, 1, DSLASH_BLOCK, 0};
     hipError_t e = hipSuccess;
     for (int zp : zps)
@@ -2026,7 +2046,6 @@ int cl2_autotune_dks(cl2_ctx* c, const void* gauge, int fmt, double* best_ms, in
                     bt   = cl2_hop_tuning{zp, x, 1, 1, sh.first, sh.second};
                 }
             }
-    c->tune_manual = manual;
     if (e != hipSuccess) {
         c->tuned.erase(key);
         CL2_HIP(c, e);

@@ -118,9 +118,6 @@ __host__ __device__ constexpr int unit_conj(int u)
 {
     return u == PI ? MI : (u == MI ? PI : u);
 }
-/* block shape of the wave-per-hop kernels: 64 sites, one wave for each of the eight hops */
-constexpr int SPLIT_SITES = 64, SPLIT_BLOCK = 8 * SPLIT_SITES;
-
 template<typename R>
 struct Su3 {
     Cx<R> e[3][3];

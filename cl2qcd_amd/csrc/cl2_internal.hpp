@@ -17,7 +17,7 @@ struct cl2_hop_tuning {
     int xcd;      // XCD-contiguous block assignment
     int rb;       // right-hand sides per thread of the multi-RHS kernel
     int lds;      // 1: the multi-RHS kernel stages each site's links and neighbour indices in LDS once
-    int block;    // threads per block of the single-field kernel
+    int block;    // sites per block of the single-field kernel: 128, 256 or 512 threads, one each, or SPLIT_SITES
     int occ;      // register budget of the single-field kernel: 0 (<= 2 waves per SIMD, hop pairs), 1 (1 wave,
                   // four hops in flight), 4 (>= 4 waves, one hop at a time); -1: the format's default
 };
@@ -36,14 +36,14 @@ struct cl2_ctx {
     void** ptr_table = nullptr;  // device copy of the field-pointer table of the multi-shift update (2 x 64)
     std::vector<void*> ptr_table_host;  // what ptr_table holds
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
-    int tune_zplanes = -1;  // z-planes per slab of the hopping kernels (-1: heuristic, 0: identity order)
-    int tune_xcd     = 1;   // XCD-contiguous block assignment
-    int tune_mrhs_rb = 0;   // right-hand sides per thread of the multi-RHS hopping kernel (0: by format)
-    int tune_block   = 256; // threads per block of the single-field hopping kernel
-    int tune_occ     = -1;  // register budget of the single-field hopping kernel (-1: the format's default)
-    int tune_mrhs_lds = 1;  // multi-RHS hopping kernel: links and neighbour indices staged in LDS per site
-    int tune_mrhs_off32 = 1;  // staged multi-RHS kernel: FP64 gathers with 32-bit offsets where they fit
-    bool tune_manual = false;  // set by cl2_tune_set: the values above override autotuned ones
+    // launch shapes set by hand (cl2_tune_set); -1 (0 for mrhs_rb and block): left to the autotuner and the size rules
+    int tune_zplanes  = -1;  // z-planes per slab of the hopping kernels (0: identity order)
+    int tune_xcd      = -1;  // XCD-contiguous block assignment
+    int tune_mrhs_rb  = 0;   // right-hand sides per thread of the multi-RHS hopping kernel
+    int tune_mrhs_lds = -1;  // multi-RHS hopping kernel: links and neighbour indices staged in LDS per site
+    int tune_block    = 0;   // sites per block of the single-field hopping kernel
+    int tune_occ      = -1;  // its register budget
+    int tune_mrhs_off32 = 1; // staged multi-RHS kernel: FP64 gathers with 32-bit offsets where they fit
     std::map<std::pair<int, int>, cl2_hop_tuning> tuned;  // (link format, right-hand sides) -> autotuned shape
     std::string err;
 };
@@ -62,8 +62,8 @@ inline unsigned blocks_for(size_t n, int block)
     return (unsigned)((n + block - 1) / block);
 }
 
-/* launch shape for (format, right-hand sides): manual settings, else the autotuned entry, else the
- * measured defaults */
+/* launch shape for (format, right-hand sides): what of it is set by hand over the measured defaults, else the autotuned
+ * entry, else the defaults */
 cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs);
 /* work order of the hopping kernels for this context's lattice and a launch shape */
 WorkMap work_map(const cl2_ctx* c, int block, int nrhs, const cl2_hop_tuning& t);

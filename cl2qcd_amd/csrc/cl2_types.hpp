@@ -69,6 +69,9 @@ struct WorkMap {
     uint32_t plane;    // eo sites of a z-plane (row != 0)
 };
 
+/* block shape of the wave-per-hop kernels: 64 sites, one wave for each of the eight hops */
+constexpr int SPLIT_SITES = 64, SPLIT_BLOCK = 8 * SPLIT_SITES;
+
 /* Epilogues fused into the Wilson hopping kernel. */
 enum DslashEpilogue : int {
     EPI_PLAIN = 0,  // out = D in                          (dslash_eo)
@@ -103,7 +106,7 @@ struct DslashArgs {
     int nrhs;  // right-hand sides per launch (fields [12][Veo][nrhs]); 1 for single fields
     int rb;    // right-hand sides per thread of the multi-RHS kernel
     int lds;   // multi-RHS kernel with one right-hand side per thread: 1 stages links and neighbour indices in LDS
-    int block; // threads per block of the single-field kernel (128, 256 or 512; SPLIT_SITES: the wave-per-hop kernel)
+    int block; // sites per block of the single-field kernel (128, 256 or 512; SPLIT_SITES: the wave-per-hop kernel)
     int occ;   // register budget of the single-field kernel: 0 (<= 2 waves per SIMD), 1 (1 wave), 4 (>= 4 waves)
     int per_rhs;  // the operator differs per right-hand side (DslashRhsArgs)
 };

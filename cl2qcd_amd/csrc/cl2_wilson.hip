@@ -759,7 +759,11 @@ static bool wave_per_hop(int fmt, uint32_t veo)
 
 cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs)
 {
-    if (!c->tune_manual) {
+    // the keys that shape this launch: a multi-RHS key leaves the single-field kernel as it is, and the other way round
+    const bool by_hand = c->tune_zplanes >= 0 || c->tune_xcd >= 0 ||
+                         (nrhs == 1 ? c->tune_block > 0 || c->tune_occ >= 0
+                                    : c->tune_mrhs_rb > 0 || c->tune_mrhs_lds >= 0);
+    if (!by_hand) {
         auto it = c->tuned.find({fmt, nrhs});
         if (it != c->tuned.end()) return it->second;
     }
@@ -768,13 +772,16 @@ cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs)
     const int occ = c->tune_occ >= 0
                         ? c->tune_occ
                         : ((fmt == GAUGE_F64_18 || fmt == GAUGE_F64_12) ? 1 : (fmt == GAUGE_F32_12 ? 2 : 0));
-    cl2_hop_tuning t{c->tune_zplanes, c->tune_xcd, c->tune_mrhs_rb, c->tune_mrhs_lds, c->tune_block, occ};
-    if (!c->tune_manual && nrhs == 1 && wave_per_hop(fmt, c->g.veo)) t.block = SPLIT_SITES;
+    // the wave-per-hop kernel has no register budgets: one set by hand asks for the other kernel
+    const bool split = nrhs == 1 && c->tune_occ < 0 && wave_per_hop(fmt, c->g.veo);
+    const int block  = c->tune_block > 0 ? c->tune_block : (split ? SPLIT_SITES : DSLASH_BLOCK);
     // Wilson fields that stay in the L2s anyway run in site order instead of slabs (slabs / site order, dslash_eo in
     // us: FP64 16^3x32 19.4 / 18.6, 20^3x40 48.1 / 47.9; FP32 16^3x32 9.5 / 8.6; FP16 7.1 / 7.0, its operators 7.8 /
     // 7.4; but FP64 24^3x48 94.5 / 96.4; the staggered and multi-RHS kernels are no faster that way)
-    if (!c->tune_manual && nrhs == 1 && !(fmt & DKS_TUNING_KEY) && c->g.veo <= 200000) t.zplanes = 0;
-    return t;
+    const bool site_order = nrhs == 1 && !(fmt & DKS_TUNING_KEY) && c->g.veo <= 200000;
+    const int zplanes     = c->tune_zplanes >= 0 ? c->tune_zplanes : (site_order ? 0 : -1);
+    return cl2_hop_tuning{zplanes, c->tune_xcd != 0, c->tune_mrhs_rb, c->tune_mrhs_lds >= 0 ? c->tune_mrhs_lds : 1, block,
+                          occ};
 }
 
 WorkMap work_map(const cl2_ctx* c, int block, int nrhs, const cl2_hop_tuning& t)

@@ -458,12 +458,14 @@ int cl2_cg_beta(cl2_ctx* ctx, double* mbeta, double* r2, const double* norms);
  *       (-1 by lattice size and format: small lattices in lexicographic order, large multi-RHS blocks in slabs
  *       that also split y; 0 lexicographic order, else a divisor of ns);
  *       "hop.xcd" -- 1: give each XCD a contiguous range of blocks, 0: hardware round robin;
- *       "hop.block" -- threads per block of the single-field hopping kernel (128, 256, 512);
+ *       "hop.block" -- sites per block of the single-field hopping kernel: 128, 256 or 512 threads with a site each,
+ *       64: the kernel of small lattices with eight waves per 64 sites, a hop each (Wilson fields; the staggered
+ *       kernel takes 256), 0 by lattice size and format;
  *       "hop.occupancy" -- its register budget: 0 (<= 2 waves per SIMD, the two hops of a direction in
  *       flight), 1 (one wave per SIMD, four hops in flight), 2 (<= 2 waves per SIMD with four hops in
  *       flight; FP32 links, else as 0), 4 (one hop at a time: at least 4 waves per SIMD for FP32 links, the
  *       compiler's choice for FP16, else as 0), -1 the format's default (1 for FP64 links, 2 for FP32, 0 for
- *       FP16);
+ *       FP16).  A budget set without "hop.block" means blocks of 256;
  *       "mrhs.rb" -- right-hand sides per thread of the multi-right-hand-side kernel (0: by format, 1, 2, 4);
  *       "mrhs.lds" -- with one right-hand side per thread, 1 (default): a block computes each site's neighbour
  *       indices and loads its links once into LDS for all its right-hand-side threads (16 sites per block for
@@ -472,17 +474,24 @@ int cl2_cg_beta(cl2_ctx* ctx, double* mbeta, double* r2, const double* norms);
  *       "mrhs.off32" -- 1 (default): the staged kernel's FP64 neighbour gathers use a scalar base per spinor
  *       component and 32-bit lane offsets while Veo * nrhs * 16 bytes < 4 GiB (beyond that, and with 0,
  *       64-bit offsets and one-size staged blocks).
- * Every setting changes only which thread computes which site and when: results are bit identical. */
+ * A key set by hand (to a value that is not its "by size" or "by format" one) puts the autotuned shape of the
+ * launches that it shapes aside; the keys that are not set keep their rules.  "hop." keys shape single-field
+ * launches, "mrhs." keys multi-RHS ones, "hop.zplanes" and "hop.xcd" both.
+ * Every setting changes only which thread computes which site and when: fields are bit identical.  The norms of
+ * the fused steps are summed in the launch's order, so they agree to rounding.
+ * cl2_tune_get returns what is set.  It also answers "hop.block.f64_18", ".f64_12", ".f32_12" and ".f16_12": the
+ * sites per block of a single-field Wilson launch with such links now (set, autotuned or by rule). */
 int cl2_tune_set(cl2_ctx* ctx, const char* key, long value);
 long cl2_tune_get(const cl2_ctx* ctx, const char* key);
 
 /* No counterpart in the reference (which fixes work-group sizes per device in hardware/device.cpp:286-334):
  * autotune the hopping kernel's launch shape for (format, nrhs) on this context -- z-planes per slab, XCD
- * mapping, right-hand sides per thread, and for single fields the block size (128, 256, 512) and register
+ * mapping, right-hand sides per thread, and for single fields the kernel, its block size and register
  * budget -- by timing every candidate on scratch fields with the given gauge field; the fastest is kept for
  * later launches (unless cl2_tune_set fixed the shape) and returned.  occupancy: the register budget, as
  * the "hop.occupancy" key of cl2_tune_set; rhs_per_thread: 1, 2 or 4, or -1 / -2 for one right-hand side per
- * thread with the links staged in LDS ("mrhs.lds" 1 / 2).  Output pointers may be null. */
+ * thread with the links staged in LDS ("mrhs.lds" 1 / 2); block: threads per block (512 for the kernel with a wave
+ * per hop, which cl2_tune_get("hop.block.<format>") tells from blocks of 512 sites).  Output pointers may be null. */
 int cl2_autotune_dslash(cl2_ctx* ctx, const void* gauge, int format, int nrhs, double* best_ms, int* zplanes,
                         int* xcd, int* rhs_per_thread, int* block, int* occupancy);
 

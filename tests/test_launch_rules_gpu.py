@@ -302,3 +302,32 @@ def test_f64_12_gather_order_keeps_the_bits(ns, nt, block):
             got.append(b.download())
         for x, y in zip(got[:3], got[3:]):
             assert np.array_equal(x, y)
+
+
+def test_keys_set_by_hand_shape_only_their_launches():
+    with abi.Context(8, 8, theta_t=1.0) as ctx:
+        block = lambda: ctx.lib.cl2_tune_get(ctx.handle, b"hop.block.f64_18")
+        assert block() == 64  # the wave-per-hop kernel of small lattices
+        for key, value in ((b"mrhs.lds", 1), (b"mrhs.lds", 0), (b"mrhs.rb", 2), (b"hop.xcd", 1), (b"hop.zplanes", 2)):
+            ctx.tune_set(key, value)
+            assert block() == 64
+        for key, value, expect in ((b"hop.block", 128, 128), (b"hop.block", 0, 64), (b"hop.occupancy", 1, 256),
+                                   (b"hop.block", 64, 64), (b"hop.occupancy", -1, 64)):
+            ctx.tune_set(key, value)
+            assert block() == expect
+        assert ctx.lib.cl2_tune_get(ctx.handle, b"hop.block") == 64
+        with pytest.raises(abi.Cl2Error):
+            ctx.tune_set(b"hop.block", 100)
+
+
+def test_autotuner_times_the_default_kernel():
+    # 8^4, FP64: the wave-per-hop kernel, which is the default there, takes 2/3 of the time of the next shape
+    with abi.Context(8, 8, theta_t=1.0) as ctx:
+        gf = ctx.gauge(seed=3, epsilon=0.35)
+        out = [ctypes.c_int() for _ in range(5)]
+        ms = ctypes.c_double()
+        ctx.autotune_dslash(gf.ptr, abi.GAUGE_F64_18, 1, ctypes.byref(ms), *[ctypes.byref(o) for o in out])
+        assert ctx.lib.cl2_tune_get(ctx.handle, b"hop.block.f64_18") == 64
+        assert out[3].value == 512  # its threads
+        ctx.tune_set(b"mrhs.lds", 2)  # another launch's key: the tuned shape stays
+        assert ctx.lib.cl2_tune_get(ctx.handle, b"hop.block.f64_18") == 64
