@@ -738,21 +738,27 @@ __global__ __launch_bounds__(BLOCK) void k_sitediag(vec2<R>* __restrict__ out, c
     store_spinor<R>(out, S, i, v);
 }
 
-/* whether a lattice of veo eo sites takes the wave-per-hop kernel for links of format fmt (default shapes; one
- * thread per site / wave per hop in us per dslash_eo, one run):
- *   FP64  8^4 7.6 / 4.8, 12^3x20 11.7 / 9.0, 14^3x22 13.9 / 11.3, but 14^3x40 17.0 / 19.7, 16^3x32 19.3 / 20.9, where
- *         the 256-thread blocks of the other kernel fill the chip and its fewer bytes in LDS count;
- *   FP32  8^4 5.7 / 4.7, 14^3x22 7.7 / 5.1, 16^3x24 8.6 / 7.8, but 14^3x40 8.2 / 8.5, 16^3x32 9.5 / 9.8 (one block per
- *         compute unit); beyond, as long as links and spinors fit the Infinity Cache, again 18^3x34 14.2 / 13.7,
- *         20^3x40 21.6 / 19.5, 24^3x48 38.8 / 35.8, and then 28^3x56 69.0 / 69.8, 32^3x64 112 / 114;
- *   FP16  8^4 5.0 / 4.8, 14^3x22 6.6 / 4.9, 14^3x40 6.9 / 6.5, 16^3x32 7.1 / 7.3, 20^3x40 12.9 / 13.8. */
+/* whether a lattice of veo eo sites takes the wave-per-hop kernel for links of format fmt.  The limits are where it
+ * stops being the faster one, or as fast, in each way of running: on one stream, where a launch has the device to
+ * itself, and (in brackets) with three contexts at work, which fill it.  There its half spinors in LDS count from
+ * about 28,000 FP64 or 50,000 FP32 and FP16 sites on.  Thread per site / wave per hop in us, QplusQminus_eo of four
+ * hopping terms, both in site order; FP16: a pass of four CG steps:
+ *   F64_18  8^4 37.3 / 19.9 (18.1 / 15.2), 12^3x20 51.4 / 38.7 (23.9 / 22.4), 14^3x20 57.8 / 46.4 (31.5 / 33.0; 33.2
+ *           before either kernel's present order), but 14^3x26 59.4 / 60.9 (40.8 / 42.5), 16^3x24 63.5 / 72.3
+ *   F64_12  8^4 32.6 / 18.6 (16.0 / 15.2), 12^3x20 42.8 / 31.3 (19.1 / 17.9), 12^3x28 45.3 / 34.4 (24.3 / 24.7), but
+ *           14^3x22 48.7 / 38.8 (28.0 / 29.5), 14^3x26 49.1 / 50.7 (32.5 / 33.9)
+ *   F32     8^4 24.4 / 15.0 (15.5 / 15.5), 14^3x22 33.0 / 23.0 (19.6 / 18.2), 16^3x24 34.8 / 31.2 (23.6 / 23.9), but
+ *           14^3x40 35.6 / 36.2 (26.3 / 27.0); 18^3x34 60.9 / 57.9 (43.5 / 45.6) and 24^3x48 165 / 151 (141 / 150) gain
+ *           on one stream and lose on three
+ *   F16     12^3x20 189 / 167 (120 / 121), 16^3x24 212 / 199 (112 / 115), but 14^3x40 215 / 217 (109 / 118), 18^3x34
+ *           278 / 303 (162 / 186) */
 static bool wave_per_hop(int fmt, uint32_t veo)
 {
     switch (fmt) {
-        case GAUGE_F64_18:
-        case GAUGE_F64_12: return veo <= 40000;
-        case GAUGE_F32_12: return veo <= 50000 || (veo >= 90000 && veo <= 400000);
-        case GAUGE_F16_12: return veo <= 60000;
+        case GAUGE_F64_18: return veo <= 28672;
+        case GAUGE_F64_12: return veo <= 24576;
+        case GAUGE_F32_12:
+        case GAUGE_F16_12: return veo <= 50000;
         default: return false;  // the staggered kernels have no such variant
     }
 }

@@ -331,3 +331,12 @@ def test_autotuner_times_the_default_kernel():
         assert out[3].value == 512  # its threads
         ctx.tune_set(b"mrhs.lds", 2)  # another launch's key: the tuned shape stays
         assert ctx.lib.cl2_tune_get(ctx.handle, b"hop.block.f64_18") == 64
+
+
+@pytest.mark.parametrize("ns,nt,blocks", [(14, 20, (64, 256, 64, 64)), (14, 22, (256, 256, 64, 64)),
+                                          (16, 24, (256, 256, 64, 64)), (14, 40, (256,) * 4), (20, 40, (256,) * 4)])
+def test_wave_per_hop_limits(ns, nt, blocks):
+    # beyond them the kernel is slower where the device is full: one such limit per format
+    with abi.Context(ns, nt) as ctx:
+        got = tuple(ctx.lib.cl2_tune_get(ctx.handle, b"hop.block." + f) for f in (b"f64_18", b"f64_12", b"f32_12", b"f16_12"))
+        assert got == blocks
