@@ -1865,8 +1865,10 @@ long cl2_tune_get(const cl2_ctx* c, const char* key)
     if (k == "hop.occupancy") return c->tune_occ;
     const char* formats[] = {"f64_18", "f64_12", "f32_12", "f16_12"};
     const int numbers[]   = {CL2_GAUGE_F64_18, CL2_GAUGE_F64_12, CL2_GAUGE_F32_12, CL2_GAUGE_F16_12};
-    for (int f = 0; f < 4; ++f)
+    for (int f = 0; f < 4; ++f) {
         if (k == std::string("hop.block.") + formats[f]) return hop_tuning(c, numbers[f], 1).block;
+        if (k == std::string("hop.zplanes.") + formats[f]) return hop_tuning(c, numbers[f], 1).zplanes;
+    }
     return -2;
 }
 

@@ -781,13 +781,19 @@ cl2_hop_tuning hop_tuning(const cl2_ctx* c, int fmt, int nrhs)
     // the wave-per-hop kernel has no register budgets: one set by hand asks for the other kernel
     const bool split = nrhs == 1 && c->tune_occ < 0 && wave_per_hop(fmt, c->g.veo);
     const int block  = c->tune_block > 0 ? c->tune_block : (split ? SPLIT_SITES : DSLASH_BLOCK);
-    // Wilson fields that stay in the L2s anyway run in site order instead of slabs (slabs / site order, dslash_eo in
-    // us: FP64 16^3x32 19.4 / 18.6, 20^3x40 48.1 / 47.9; FP32 16^3x32 9.5 / 8.6; FP16 7.1 / 7.0, its operators 7.8 /
-    // 7.4; but FP64 24^3x48 94.5 / 96.4; the staggered and multi-RHS kernels are no faster that way)
-    const bool site_order = nrhs == 1 && !(fmt & DKS_TUNING_KEY) && c->g.veo <= 200000;
+    // Small Wilson fields run in site order instead of slabs: where three t-slices of spinors stay in an XCD's L2 (2.3
+    // MB of FP64 at 20^3) a slab saves nothing and its edges cost.  Slabs / site order, QplusQminus_eo in us on one
+    // stream (three contexts at once in brackets):
+    //   F64_18  8^3x96 46.5 / 37.8 (29.2 / 28.0), 16^3x24 64.7 / 63.5 (55.5 / 54.7), 16^3x64 157 / 152 (147 / 145), but
+    //           16^3x96 229 / 221 (221 / 229), 24^3x24 201 / 205 (192 / 202), 32^3x8 148 / 168 (145 / 153)
+    //   F64_12  16^3x24 55.5 / 53.6 (45.8 / 44.9), but 16^3x40 103 / 99 (71.8 / 73.1), 24^3x24 167 / 173 (146 / 157)
+    //   F32     16^3x32 41.0 / 37.6 (29.3 / 28.7), but 24^3x8 35.7 / 39.3 (26.0 / 26.9); FP16 likewise
+    // The staggered and multi-RHS kernels are no faster that way
+    const bool site_order = nrhs == 1 && !(fmt & DKS_TUNING_KEY) && c->g.ns <= 20 &&
+                            c->g.veo <= (fmt == GAUGE_F64_12 ? 60000u : 150000u);
     const int zplanes     = c->tune_zplanes >= 0 ? c->tune_zplanes : (site_order ? 0 : -1);
-    return cl2_hop_tuning{zplanes, c->tune_xcd != 0, c->tune_mrhs_rb, c->tune_mrhs_lds >= 0 ? c->tune_mrhs_lds : 1, block,
-                          occ};
+    const int lds         = c->tune_mrhs_lds >= 0 ? c->tune_mrhs_lds : 1;
+    return cl2_hop_tuning{zplanes, c->tune_xcd != 0, c->tune_mrhs_rb, lds, block, occ};
 }
 
 WorkMap work_map(const cl2_ctx* c, int block, int nrhs, const cl2_hop_tuning& t)

@@ -479,8 +479,9 @@ int cl2_cg_beta(cl2_ctx* ctx, double* mbeta, double* r2, const double* norms);
  * launches, "mrhs." keys multi-RHS ones, "hop.zplanes" and "hop.xcd" both.
  * Every setting changes only which thread computes which site and when: fields are bit identical.  The norms of
  * the fused steps are summed in the launch's order, so they agree to rounding.
- * cl2_tune_get returns what is set.  It also answers "hop.block.f64_18", ".f64_12", ".f32_12" and ".f16_12": the
- * sites per block of a single-field Wilson launch with such links now (set, autotuned or by rule). */
+ * cl2_tune_get returns what is set.  It also answers "hop.block.f64_18", ".f64_12", ".f32_12" and ".f16_12", the
+ * sites per block of a single-field Wilson launch with such links now (set, autotuned or by rule), and
+ * "hop.zplanes." likewise (-1: slabs by lattice size). */
 int cl2_tune_set(cl2_ctx* ctx, const char* key, long value);
 long cl2_tune_get(const cl2_ctx* ctx, const char* key);
 

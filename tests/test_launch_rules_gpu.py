@@ -340,3 +340,11 @@ def test_wave_per_hop_limits(ns, nt, blocks):
     with abi.Context(ns, nt) as ctx:
         got = tuple(ctx.lib.cl2_tune_get(ctx.handle, b"hop.block." + f) for f in (b"f64_18", b"f64_12", b"f32_12", b"f16_12"))
         assert got == blocks
+
+
+@pytest.mark.parametrize("ns,nt,planes", [(16, 24, (0, 0)), (16, 64, (0, -1)), (20, 36, (0, -1)), (16, 96, (-1, -1)),
+                                          (24, 8, (-1, -1)), (32, 4, (-1, -1))])
+def test_site_order_limits(ns, nt, planes):
+    # lexicographic order only where t-slices are small, whatever the number of sites
+    with abi.Context(ns, nt) as ctx:
+        assert tuple(ctx.lib.cl2_tune_get(ctx.handle, b"hop.zplanes." + f) for f in (b"f64_18", b"f64_12")) == planes
