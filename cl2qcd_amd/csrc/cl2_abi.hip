@@ -1868,6 +1868,21 @@ long cl2_tune_get(const cl2_ctx* c, const char* key)
     for (int f = 0; f < 4; ++f) {
         if (k == std::string("hop.block.") + formats[f]) return hop_tuning(c, numbers[f], 1).block;
         if (k == std::string("hop.zplanes.") + formats[f]) return hop_tuning(c, numbers[f], 1).zplanes;
+        for (int n : {2, 4, 8, 12, 16}) {
+            const std::string tail = std::string(formats[f]) + "." + std::to_string(n);
+            const int bytes        = numbers[f] == CL2_GAUGE_F32_12 ? 4 : 8;
+            if (k == "stagg.pairs." + tail) return dks_pairs(c, numbers[f], n);
+            if (k == "mrhs.slab." + tail) {
+                const cl2_hop_tuning t = hop_tuning(c, numbers[f], n);
+                if (numbers[f] == CL2_GAUGE_F16_12 || t.rb > 1 || !t.lds) return 0;
+                return work_map_mrhs(c, mrhs_sites_per_block(n, t.lds), bytes, 24u * n, t).row;
+            }
+            if (k == "stagg.slab." + tail && numbers[f] != CL2_GAUGE_F16_12) {
+                const cl2_hop_tuning t = hop_tuning(c, numbers[f] | DKS_TUNING_KEY, n);
+                const int sites        = dks_pairs(c, numbers[f], n) ? 32 : mrhs_sites_per_block(n, 1);
+                return work_map_mrhs(c, sites, bytes, 6u * n, t).row;
+            }
+        }
     }
     return -2;
 }

@@ -85,6 +85,8 @@ int mrhs_sites_per_block(int nrhs, int lds);
 /* the staged multi-RHS kernel's FP64 gathers use 32-bit byte offsets within a component: veo * nrhs complex
  * numbers of complex_bytes each must stay below 4 GiB, else it takes 64-bit offsets (and lds 1 only) */
 bool mrhs_offsets_narrow(uint32_t veo, int nrhs, size_t complex_bytes);
+/* whether 16-byte aligned staggered blocks take the kernel with two right-hand sides per thread */
+bool dks_pairs(const cl2_ctx* c, int format, int nrhs);
 /* right-hand-side counts with a compiled multi-RHS hopping kernel */
 bool supported_nrhs(int n);
 

@@ -446,6 +446,11 @@ static void dks_weights(cl2_ctx* c, DksArgs& a)
     }
 }
 
+bool dks_pairs(const cl2_ctx* c, int format, int nrhs)
+{
+    return format == GAUGE_F32_12 && nrhs >= 8 && mrhs_offsets_narrow(c->g.veo, nrhs, sizeof(float2));
+}
+
 hipError_t launch_dks_mrhs(cl2_ctx* c, void* out, const void* in, const void* gauge, int format, int evenodd, int nrhs,
                            const void* x, const double* coef, double2* norm_partials, const void* own, void* cg_r,
                            const double* cg_alpha, unsigned* nblocks)
@@ -463,8 +468,10 @@ hipError_t launch_dks_mrhs(cl2_ctx* c, void* out, const void* in, const void* ga
     a.cg_alpha      = cg_alpha;
     for (int r = 0; r < 16; ++r) a.coef[r] = (x && r < nrhs) ? coef[r] : 0.;
     dks_weights(c, a);
-    const cl2_hop_tuning t = hop_tuning(c, format | DKS_TUNING_KEY, 1);
-    const bool pairs = format == GAUGE_F32_12 && mrhs_offsets_narrow(c->g.veo, nrhs, sizeof(float2)) &&
+    // the block's own shape: a slab that the autotuner found for one field is a poor one for many (16 right-hand sides at
+    // 48^3x12: 3278 us per four CG steps, 3339 with it; 12 at 40^3x20 2500 and 2625)
+    const cl2_hop_tuning t = hop_tuning(c, format | DKS_TUNING_KEY, nrhs);
+    const bool pairs = dks_pairs(c, format, nrhs) &&
                        ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(in) |
                          reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(own) |
                          reinterpret_cast<uintptr_t>(cg_r)) & 15u) == 0;

@@ -481,7 +481,9 @@ int cl2_cg_beta(cl2_ctx* ctx, double* mbeta, double* r2, const double* norms);
  * the fused steps are summed in the launch's order, so they agree to rounding.
  * cl2_tune_get returns what is set.  It also answers "hop.block.f64_18", ".f64_12", ".f32_12" and ".f16_12", the
  * sites per block of a single-field Wilson launch with such links now (set, autotuned or by rule), and
- * "hop.zplanes." likewise (-1: slabs by lattice size). */
+ * "hop.zplanes." likewise (-1: slabs by lattice size); and of multi-RHS launches "mrhs.slab.<format>.<nrhs>" (Wilson)
+ * and "stagg.slab.<format>.<nrhs>", the eo sites of a z-plane in a slab that holds part of y (0: whole planes), and
+ * "stagg.pairs.<format>.<nrhs>", 1 where 16-byte aligned blocks take two right-hand sides per thread. */
 int cl2_tune_set(cl2_ctx* ctx, const char* key, long value);
 long cl2_tune_get(const cl2_ctx* ctx, const char* key);
 
@@ -497,7 +499,7 @@ int cl2_autotune_dslash(cl2_ctx* ctx, const void* gauge, int format, int nrhs, d
                         int* xcd, int* rhs_per_thread, int* block, int* occupancy);
 
 /* No counterpart in the reference: the same autotuning for the staggered hopping kernel (cl2_D_KS_eo and the
- * staggered operators built on it) with links of the given format (FP64 or FP32): z-planes per slab, XCD
+ * staggered operators on single fields built on it) with links of the given format (FP64 or FP32): z-planes per slab, XCD
  * mapping, block size and register budget. */
 int cl2_autotune_dks(cl2_ctx* ctx, const void* gauge, int format, double* best_ms, int* zplanes, int* xcd,
                      int* block, int* occupancy);

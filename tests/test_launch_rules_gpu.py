@@ -348,3 +348,16 @@ def test_site_order_limits(ns, nt, planes):
     # lexicographic order only where t-slices are small, whatever the number of sites
     with abi.Context(ns, nt) as ctx:
         assert tuple(ctx.lib.cl2_tune_get(ctx.handle, b"hop.zplanes." + f) for f in (b"f64_18", b"f64_12")) == planes
+
+
+def test_single_field_autotuning_leaves_staggered_blocks_alone():
+    # a 28^3 block has slabs of 7 planes and 14 rows: whole planes that the autotuner finds for one field must not replace them
+    with abi.Context(28, 12, theta_t=1.0) as ctx:
+        gf = ctx.gauge(seed=3, epsilon=0.35).converted(abi.GAUGE_F32_12)
+        slab = lambda: ctx.lib.cl2_tune_get(ctx.handle, b"stagg.slab.f32_12.16")
+        before = slab()
+        assert 0 < before < 28 * 14
+        ctx.autotune_dks(gf.ptr, abi.GAUGE_F32_12, None, None, None, None, None)
+        assert slab() == before
+        ctx.tune_set(b"hop.zplanes", 7)  # by hand: as set
+        assert slab() == 0
