@@ -222,7 +222,7 @@ struct RhsParams {
 int run_dslash(cl2_ctx* c, void* out, const void* in, const void* x, const void* gauge, int fmt, int evenodd,
                double kappa, int epilogue, const double f1[2], const double f2[2], double scale, int gamma5,
                int nrhs = 1, const RhsParams* pr = nullptr, double* norm_res = nullptr, void* cg_r = nullptr,
-               const double* cg_alpha = nullptr, const SumTail* tail = nullptr)
+               const double* cg_alpha = nullptr, const BlockSumTail* tail = nullptr)
 {
     CL2_REQUIRE(c, valid_fmt(fmt), "unknown gauge format");
     CL2_REQUIRE(c, supported_nrhs(nrhs), "unsupported number of right-hand sides (1, 2, 4, 8, 12 or 16)");
@@ -344,7 +344,7 @@ void tm_factors(int variant, double mubar, double f1[2], double f2[2], double* s
 int run_aee(cl2_ctx* c, void* out, const void* in, void* tmp, const void* gauge, int fmt, int action, double kappa,
             double mubar, bool minus, bool gamma5, int nrhs = 1, const double* kappas = nullptr,
             const double* mubars = nullptr, double* norm_res = nullptr, void* cg_r = nullptr,
-            const double* cg_alpha = nullptr, const SumTail* tail = nullptr)
+            const double* cg_alpha = nullptr, const BlockSumTail* tail = nullptr)
 {
     double f1[2], f2[2], s;
     int rc;
@@ -965,7 +965,7 @@ int cl2_fermionmatrix_eo_cg_step(cl2_ctx* c, int op, void* r, const void* p, con
     CL2_REQUIRE(c, r != t0 && r != t1 && p != t0 && p != t1, "tmp must not alias r or p");
     // t1 = Qminus p with pAp = |t1|^2 and alpha = r2 / pAp by the block that finishes that sum; then Qplus t1 is folded
     // into r <- r - alpha Qplus t1
-    SumTail tail{};
+    BlockSumTail tail{};
     tail.kind  = TAIL_RATIO;
     tail.r2    = r2;
     tail.alpha = alpha;
@@ -995,7 +995,7 @@ int cl2_fermionmatrix_eo_mrhs_cg_step(cl2_ctx* c, int op, void* r, const void* p
     void* t0        = tmp;
     void* t1        = static_cast<char*>(tmp) + fb;
     CL2_REQUIRE(c, r != t0 && r != t1 && p != t0 && p != t1, "tmp must not alias r or p");
-    SumTail tail{};
+    BlockSumTail tail{};
     tail.kind   = TAIL_ALPHA;
     tail.r2     = r2;
     tail.active = active;
@@ -1430,7 +1430,7 @@ int cl2_MdagM_eo_mrhs_cg_step(cl2_ctx* c, void* r, const void* p, const void* ga
     CL2_REQUIRE(c, upper_left == CL2_EVEN || upper_left == CL2_ODD, "upper_left must be CL2_EVEN or CL2_ODD");
     CL2_REQUIRE(c, r && p && gauge && tmp && r2 && active && pAp && alpha && norms, "null pointer");
     CL2_REQUIRE(c, r != p && tmp != p && tmp != r, "r, p and tmp must be different blocks");
-    SumTail tail{};
+    BlockSumTail tail{};
     tail.kind   = TAIL_ALPHA_MDAGM;
     tail.r2     = r2;
     tail.active = active;

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void k_block_dot(const void* x, const void* y,
 template<int BLOCK, bool WIDE, bool TAIL>
 __global__ __launch_bounds__(BLOCK) void k_block_reduce2(const double2* partials, unsigned nb, double* res,
                                                          int out_kind,
-                                                         typename std::conditional<TAIL, SumTail, NoTail>::type tail)
+                                                         typename std::conditional<TAIL, BlockSumTail, NoTail>::type tail)
 {
     __shared__ double lds[2 * BLOCK / 64];
     const double2 s = block_sum2<BLOCK>(strided_sum<BLOCK, WIDE>(partials + (size_t)blockIdx.x * nb, nb), lds);
@@ -377,11 +377,11 @@ static BlockShape block_shape(cl2_ctx* c, size_t n, int prec, int nrhs, int u, b
 constexpr int BLOCK_U_REDUCE = 4;
 
 hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, double* res, int out_kind, int nrhs,
-                                const SumTail* tail)
+                                const BlockSumTail* tail)
 {
     // The step lengths are formed by each right-hand side's own block, in any order.  Where a caller's arrays overlap,
     // one block's alpha or sum could land on what another has yet to read: a launch after all the sums forms them then
-    SumTail sums_only;
+    BlockSumTail sums_only;
     if (tail && tail->alpha) {
         auto apart = [](const double* a, int na, const double* b, int nb_) {
             const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);

@@ -157,6 +157,9 @@ struct SumTail {
     double* alpha;
     double *beta, *beta_prev, *pap;
     double m2;
+};
+/* with the lockstep steps' coefficients, 128 bytes that the launches without them do without */
+struct BlockSumTail : SumTail {
     double coef[16];
 };
 struct NoTail {
@@ -205,7 +208,7 @@ hipError_t launch_block_dot(cl2_ctx* c, double* res, const void* x, const void* 
 /* stage 2 of the per-right-hand-side reductions: block r sums partials[r * nb .. r * nb + nb) in order;
  * out_kind 0: res[2r..2r+1] = complex sum, 1: res[r] = real part */
 hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, double* res, int out_kind, int nrhs,
-                                const SumTail* tail = nullptr);
+                                const BlockSumTail* tail = nullptr);
 hipError_t launch_block_xp(cl2_ctx* c, void* x, void* p, const void* r, int prec, int nrhs, const double* alpha,
                            const double* beta, int ncomp = 12);
 hipError_t launch_block_slot(cl2_ctx* c, void* block, const void* single_in, void* single_out, int prec, int nrhs,
