@@ -8,7 +8,10 @@
 * the streaming multi-shift update agrees with numpy;
 * stage 2 of the reductions sums every one of many partials once;
 * the work order of large multi-RHS fields, slabs that split y, visits every site: site order's bits;
-* cl2_scalar_get returns what the stream wrote, on both sides of the mailbox's size.
+* cl2_scalar_get returns what the stream wrote, on both sides of the mailbox's size and of the time the host watches it,
+  and refuses what a copy refuses;
+* the lockstep steps take arrays that overlap;
+* tuning keys and the autotuner leave other launches' shapes alone, and the size rules pick what they say.
 """
 import ctypes
 
@@ -24,6 +27,12 @@ pytestmark = pytest.mark.gpu
 FORMATS = [(abi.GAUGE_F64_18, abi.F64), (abi.GAUGE_F64_12, abi.F64), (abi.GAUGE_F32_12, abi.F32),
            (abi.GAUGE_F16_12, abi.F16)]
 KAPPA, MUBAR = 0.16, 0.0016
+NAMES = {abi.GAUGE_F64_18: "f64_18", abi.GAUGE_F64_12: "f64_12", abi.GAUGE_F32_12: "f32_12", abi.GAUGE_F16_12: "f16_12"}
+
+
+def chosen(ctx, what, fmt, nrhs=None):
+    """What the launch rules pick for links of format fmt on this context."""
+    return ctx.lib.cl2_tune_get(ctx.handle, ".".join([what, NAMES[fmt]] + ([str(nrhs)] if nrhs else [])).encode())
 
 
 @pytest.mark.parametrize("phases", [dict(theta_t=1.0), dict(theta_t=1.0, theta_s=0.3, cp_im=0.2)],
@@ -37,6 +46,7 @@ def test_wave_per_hop_matches_thread_per_site(fmt, prec, ns, nt, phases):
         with abi.Context(ns, nt, **phases) as ctx:
             if block:
                 ctx.tune_set(b"hop.block", block)
+            assert chosen(ctx, "hop.block", fmt) == (block or 64)
             rng = np.random.default_rng(7)
             gf = ctx.gauge(random_su3_field(4 * O.volume(lat), 8), fmt)
             src, r0 = rng.standard_normal((ctx.veo, 24)), rng.standard_normal((ctx.veo, 24))
@@ -76,6 +86,7 @@ def test_staggered_pairs_match_single(nrhs, offset):
     ns, nt, mass = 6, 10, 0.1  # 1080 eo sites: 33 blocks of 32 sites and a rest of 24
     with abi.Context(ns, nt, theta_t=1.0) as ctx:
         lat = O.lattice(ns, nt, theta_t=1.0)
+        assert chosen(ctx, "stagg.pairs", abi.GAUGE_F32_12, nrhs) == 1  # with the aligned offset, 0
         gf = ctx.gauge(random_su3_field(4 * O.volume(lat), 3)).converted(abi.GAUGE_F32_12)
         rng = np.random.default_rng(nrhs)
         one = ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SU3VEC_EO, abi.F32)
@@ -183,6 +194,7 @@ def test_many_partial_sums():
     (abi.GAUGE_F32_12, abi.F32, 12, 12, 36), (abi.GAUGE_F32_12, abi.F32, 16, 20, 6), (abi.GAUGE_F32_12, abi.F32, 8, 18, 16)])
 def test_slabs_in_y_visit_every_site(fmt, prec, nrhs, ns, nt):
     with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        assert chosen(ctx, "mrhs.slab", fmt, nrhs) == {12: 36, 16: 64, 20: 100, 18: 0}[ns]  # rows times ns / 2
         gf = ctx.gauge(random_su3_field(4 * ns ** 3 * nt, 8), fmt)
         one = ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SPINOR_EO, prec)
         src = ctx.spinor(prec).upload(np.random.default_rng(9).standard_normal((ctx.veo, 24)))
@@ -203,6 +215,7 @@ def test_slabs_in_y_visit_every_site(fmt, prec, nrhs, ns, nt):
     (abi.GAUGE_F64_12, abi.F64, 12, 20, 16), (abi.GAUGE_F32_12, abi.F32, 16, 24, 14), (abi.GAUGE_F32_12, abi.F32, 12, 20, 30)])
 def test_staggered_slabs_in_y_visit_every_site(fmt, prec, nrhs, ns, nt):
     with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        assert chosen(ctx, "stagg.slab", fmt, nrhs) == {20: 100, 24: 144}[ns]
         gf = ctx.gauge(random_su3_field(4 * ns ** 3 * nt, 3)).converted(fmt)
         one = ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SU3VEC_EO, prec)
         src = ctx.su3vec(prec).upload(np.random.default_rng(9).standard_normal((ctx.veo, 6)))
@@ -267,6 +280,24 @@ def test_lockstep_step_with_shared_arrays(staggered, shared):
         assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
 
 
+def test_scalar_get_behind_queued_work():
+    # several milliseconds of hopping terms in front of the sum that is read: past the time the host watches the mailbox
+    with abi.Context(24, 48, theta_t=1.0) as ctx:
+        gf = ctx.gauge(seed=3, epsilon=0.0)
+        a, b, s = ctx.spinor(), ctx.spinor(), ctx.scalars(1)
+        ctx.set_cold_eo(a.ptr, abi.F64)
+        for reps in (1, 41):  # each time as many as leave the field in `b`
+            s.store([-1.0])
+            ctx.set_cold_eo(a.ptr, abi.F64)
+            for k in range(reps):
+                src, dst = (a, b) if k % 2 == 0 else (b, a)
+                ctx.dslash_eo(dst.ptr, src.ptr, gf.ptr, abi.GAUGE_F64_18, abi.EVEN if k % 2 == 0 else abi.ODD, 0.125)
+            ctx.squarenorm_eo(s.ptr, b.ptr, abi.F64)
+            early = s.get()[0]
+            ctx.sync()
+            assert early == s.get()[0] and early > 0.0
+
+
 def test_scalar_get_refuses_what_a_copy_refuses():
     # a range beyond its allocation, and host memory: errors, and the next read and the next launch are in order again
     with abi.Context(4, 4) as ctx:
@@ -301,6 +332,32 @@ def test_f64_12_gather_order_keeps_the_bits(ns, nt, block):
                                  abi.ACTION_TWISTEDMASS, KAPPA, MUBAR, tmp.ptr)
             got.append(b.download())
         for x, y in zip(got[:3], got[3:]):
+            assert np.array_equal(x, y)
+
+
+# 378 and 648 blocks, which the XCDs share in contiguous ranges, in both orders of the sites
+@pytest.mark.parametrize("planes", [0, 2])
+@pytest.mark.parametrize("ns,nt", [(12, 28), (24, 6)])
+@pytest.mark.parametrize("fmt,prec", FORMATS)
+def test_wave_per_hop_work_orders(fmt, prec, ns, nt, planes):
+    with abi.Context(ns, nt, theta_t=1.0) as ctx:
+        g18 = ctx.gauge(seed=3, epsilon=0.35)
+        gf = g18 if fmt == abi.GAUGE_F64_18 else g18.converted(fmt)
+        a, b = ctx.spinor(prec), ctx.spinor(prec)
+        a.upload(np.random.default_rng(7).standard_normal((ctx.veo, 24)))
+        tmp = ctx.buffer(2 * ctx.lib.cl2_field_bytes(ctx.handle, abi.FIELD_SPINOR_EO, prec))
+        results = []
+        for block, zp in ((64, planes), (256, 0)):
+            ctx.tune_set(b"hop.block", block)
+            ctx.tune_set(b"hop.zplanes", zp)
+            got = []
+            for evenodd in (abi.EVEN, abi.ODD):
+                ctx.dslash_eo(b.ptr, a.ptr, gf.ptr, fmt, evenodd, KAPPA)
+                got.append(b.download())
+            ctx.fermionmatrix_eo(abi.OP_QPLUSQMINUS_EO, b.ptr, a.ptr, gf.ptr, fmt, abi.ACTION_TWISTEDMASS, KAPPA, MUBAR,
+                                 tmp.ptr)
+            results.append(got + [b.download()])
+        for x, y in zip(*results):
             assert np.array_equal(x, y)
 
 
