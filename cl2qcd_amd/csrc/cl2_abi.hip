@@ -473,13 +473,11 @@ int cl2_ctx_create(cl2_ctx** out, int device, const cl2_lattice* lat)
         hipMalloc(&c->partials, c->npartials * 2 * sizeof(double)) != hipSuccess ||
         hipMalloc(&c->dscratch, 64 * sizeof(double)) != hipSuccess ||
         hipMalloc(&c->ptr_table, 128 * sizeof(void*)) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&c->mail.box), sizeof(cl2_mailbox), hipHostMallocDefault) != hipSuccess ||
         hipEventCreate(&c->ev_start) != hipSuccess || hipEventCreate(&c->ev_stop) != hipSuccess) {
         cl2_ctx_destroy(c);
         return create_fail(CL2_E_HIP, "context allocation failed");
     }
-    c->mail.box->number = 0;
-    *out                = c;
+    *out = c;
     return CL2_OK;
 }
 
@@ -853,11 +851,31 @@ static bool readable_by_kernel(cl2_ctx* c, const void* p, size_t bytes)
            capture == hipStreamCaptureStatusNone;
 }
 
+/* pinned memory for the mailbox: 12 us to get and 35 to give back, which a context that never reads a scalar does not
+ * pay (45 us to create and 75 to destroy on 8^4).  A capture on this thread, another context's, does not mind an
+ * allocation that is not recorded */
+static cl2_mailbox* allocate_mailbox()
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    cl2_mailbox* box = nullptr;
+    if (hipHostMalloc(reinterpret_cast<void**>(&box), sizeof(cl2_mailbox), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        box = nullptr;
+    }
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) (void)hipGetLastError();
+    if (box) box->number = 0;
+    return box;
+}
+
 int cl2_scalar_get(cl2_ctx* c, double* host, const double* dev, int n)
 {
     if (!c) return CL2_E_ARG;
     CL2_REQUIRE(c, dev && host && n > 0, "bad scalar get");
-    if (n > cl2_mailbox::SIZE || !readable_by_kernel(c, dev, n * sizeof(double))) {
+    if (n > cl2_mailbox::SIZE || !readable_by_kernel(c, dev, n * sizeof(double)) || !c->mail.open(allocate_mailbox)) {
         CL2_HIP(c, hipMemcpyAsync(host, dev, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         CL2_HIP(c, hipStreamSynchronize(c->stream));
         return CL2_OK;

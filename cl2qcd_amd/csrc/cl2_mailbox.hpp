@@ -19,6 +19,15 @@ class cl2_mail_reader {
   public:
     cl2_mailbox* box = nullptr;
 
+    /* the box, from allocate() at the first call that gets one; false without one */
+    template<typename Allocate>
+    bool open(Allocate&& allocate)
+    {
+        std::lock_guard<std::mutex> one_at_a_time(mutex_);
+        if (!box) box = allocate();
+        return box != nullptr;
+    }
+
     /* n <= SIZE values into host: send(number) enqueues the transfer, and where it has not come within a millisecond
      * wait() waits for everything enqueued; both return 0 or an error, which ends the read */
     template<typename Send, typename Wait>

@@ -19,7 +19,9 @@ static void deliver(uint64_t number, double v)
 int main()
 {
     cl2_mail_reader reader;
-    reader.box = &box;
+    // the box is asked for until there is one, and then no more
+    if (reader.open([] { return (cl2_mailbox*)nullptr; })) return 6;
+    if (!reader.open([] { return &box; }) || !reader.open([] { return (cl2_mailbox*)nullptr; })) return 7;
     double got = 0.;
     // one that comes at once, and one that comes while the stream is waited for
     if (reader.read(&got, 1, [](uint64_t k) { deliver(k, 1.); return 0; }, [] { return 9; }) != 0 || got != 1.) return 1;
