@@ -306,7 +306,7 @@ void k_dslash_eo(typename std::conditional<NRHS == 1, DslashArgs, DslashRhsArgs>
 
 /* ---- the hopping kernel of small lattices: a wave per hop ----
  * A lattice of a few thousand eo sites fills few compute units with one thread per site, and each of its threads then
- * works through eight hops one after the other (8.9 us for an 8^4 lattice, 8 blocks).  Here a block of eight waves
+ * works through eight hops one after the other (an 8^4 lattice has 8 blocks).  Here a block of eight waves
  * owns 64 consecutive sites of the work order and wave h computes hop h of all of them (h = 2 dir + backward: every
  * wave runs one straight piece of code, and its link and spinor loads stay contiguous); the hops' half spinors meet
  * in LDS, where waves 0..5 add up two components each in the order T, X, Y, Z, forward then backward, and apply the
