@@ -251,14 +251,14 @@ hipError_t launch_reduce_stage1(cl2_ctx* c, const void* x, const void* y, size_t
 /* stage 2: one block sums the partials in a fixed order.
  * out_kind 0: res[0] = re;  1: res = (re, im);  2: res[k] = alpha[k]^2 * re for k < nvec;
  * 3: res = (re, im, re, 0) */
-template<int BLOCK, bool WIDE, bool TAIL>
+template<int BLOCK, unsigned U, bool TAIL>
 __global__ __launch_bounds__(BLOCK) void k_reduce2(const double* __restrict__ partials, unsigned nparts, double* res,
                                                    int out_kind, const double* __restrict__ alpha, int nvec,
                                                    typename std::conditional<TAIL, SumTail, NoTail>::type tail)
 {
     __shared__ double lds[2 * BLOCK / 64];
     const double2 s =
-        block_sum2<BLOCK>(strided_sum<BLOCK, WIDE>(reinterpret_cast<const double2*>(partials), nparts), lds);
+        block_sum2<BLOCK>(strided_sum<BLOCK, U>(reinterpret_cast<const double2*>(partials), nparts), lds);
     if (threadIdx.x == 0) {
         if (out_kind == 0) {
             res[0] = s.x;
@@ -297,10 +297,10 @@ hipError_t launch_reduce_stage2(cl2_ctx* c, unsigned nparts, double* res, int ou
     auto go         = [&](auto kernel, auto t) {
         hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, c->stream, p, nparts, res, out_kind, alpha_vec, nvec, t);
     };
-    if (nparts >= WIDE_SUM_MIN(1024))
-        tail ? go(k_reduce2<1024, true, true>, *tail) : go(k_reduce2<1024, true, false>, NoTail{});
+    if (nparts >= WIDE_SUM_MIN)
+        tail ? go(k_reduce2<1024, 8, true>, *tail) : go(k_reduce2<1024, 8, false>, NoTail{});
     else
-        tail ? go(k_reduce2<1024, false, true>, *tail) : go(k_reduce2<1024, false, false>, NoTail{});
+        tail ? go(k_reduce2<1024, 1, true>, *tail) : go(k_reduce2<1024, 1, false>, NoTail{});
     return hipGetLastError();
 }
 

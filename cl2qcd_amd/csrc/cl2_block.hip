@@ -230,13 +230,13 @@ __global__ __launch_bounds__(256) void k_block_dot(const void* x, const void* y,
 
 /* stage 2: block r sums right-hand side r's nb partials; out_kind 0: res[2r..2r+1] = complex sum,
  * 1: res[r] = real part */
-template<int BLOCK, bool WIDE, bool TAIL>
+template<int BLOCK, unsigned U, bool TAIL>
 __global__ __launch_bounds__(BLOCK) void k_block_reduce2(const double2* partials, unsigned nb, double* res,
                                                          int out_kind,
                                                          typename std::conditional<TAIL, BlockSumTail, NoTail>::type tail)
 {
     __shared__ double lds[2 * BLOCK / 64];
-    const double2 s = block_sum2<BLOCK>(strided_sum<BLOCK, WIDE>(partials + (size_t)blockIdx.x * nb, nb), lds);
+    const double2 s = block_sum2<BLOCK>(strided_sum<BLOCK, U>(partials + (size_t)blockIdx.x * nb, nb), lds);
     if (threadIdx.x == 0) {
         const unsigned r = blockIdx.x;
         double2 v        = s;
@@ -398,13 +398,18 @@ hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, d
             return launch_block_cg_scalars(c, 0, tail->alpha, const_cast<double*>(tail->r2), res, tail->active, nrhs);
         }
     }
-    auto go = [&](auto kernel, auto t) {
-        hipLaunchKernelGGL(kernel, dim3(nrhs), dim3(1024), 0, c->stream, parts, nb, res, out_kind, t);
+    auto go = [&](auto kernel, unsigned threads, auto t) {
+        hipLaunchKernelGGL(kernel, dim3(nrhs), dim3(threads), 0, c->stream, parts, nb, res, out_kind, t);
     };
-    if (nb >= WIDE_SUM_MIN(1024))
-        tail ? go(k_block_reduce2<1024, true, true>, *tail) : go(k_block_reduce2<1024, true, false>, NoTail{});
+    // Many partials: 512 threads with four loads in flight (7.4 us for the 20736 per right-hand side of 16 at 48^3x12;
+    // with one load 18.6 for the 41472 that were there before).  1024 with eight hold four times the registers, and on
+    // a device that other contexts keep busy such a block waits for a compute unit to come free: two CG steps on 12 FP16
+    // right-hand sides at 30^3x22 took 2309 us with one load in flight, 2367 with those, 2297 with these (alone on the
+    // device 2222, 2187, 2184); four on 4 staggered ones at 32^3x32 918, 942, 912 (1097, 1075, 1076)
+    if (nb >= WIDE_SUM_MIN)
+        tail ? go(k_block_reduce2<512, 4, true>, 512, *tail) : go(k_block_reduce2<512, 4, false>, 512, NoTail{});
     else
-        tail ? go(k_block_reduce2<1024, false, true>, *tail) : go(k_block_reduce2<1024, false, false>, NoTail{});
+        tail ? go(k_block_reduce2<1024, 1, true>, 1024, *tail) : go(k_block_reduce2<1024, 1, false>, 1024, NoTail{});
     return hipGetLastError();
 }
 

@@ -571,19 +571,14 @@ __device__ __forceinline__ double2 block_sum2(double2 v, double* lds)
     return r;
 }
 
-/* a thread's share of n partial sums (elements threadIdx.x + k BLOCK).  WIDE, for at least WIDE_SUM_MIN partials:
- * eight loads in flight; with one load per addition the stage-2 kernels waited out the memory latency for every BLOCK partials (11.3
- * us for the 20736 of a hopping kernel at 48^3x96, 8.1 us so; per right-hand side of 16 at 48^3x12 18.6 us for
- * 41472, 7.8 us for the 20736 left there).  Fewer partials keep the short loop: the longer code costs a launch 0.5
- * us.  The order of the additions depends on n and BLOCK only. */
-constexpr unsigned WIDE_SUM_MIN(unsigned block)
-{
-    return 8 * block;
-}
-template<int BLOCK, bool WIDE>
+/* a thread's share of n partial sums (elements threadIdx.x + k BLOCK), U loads in flight: with one load per addition
+ * the stage-2 kernels waited out the memory latency for every BLOCK partials (11.3 us for the 20736 of a hopping kernel
+ * at 48^3x96, 8.1 us with 1024 threads and eight loads).  Fewer partials than WIDE_SUM_MIN keep one load: the longer
+ * code costs a launch 0.5 us.  The order of the additions depends on n, BLOCK and U only. */
+constexpr unsigned WIDE_SUM_MIN = 8192;
+template<int BLOCK, unsigned U>
 __device__ __forceinline__ double2 strided_sum(const double2* __restrict__ p, unsigned n)
 {
-    constexpr unsigned U = WIDE ? 8 : 1;
     double2 acc[U];
 #pragma unroll
     for (unsigned u = 0; u < U; ++u) acc[u] = make_double2(0., 0.);
