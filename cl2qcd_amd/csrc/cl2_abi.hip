@@ -1969,9 +1969,12 @@ int cl2_autotune_dslash(cl2_ctx* c, const void* gauge, int fmt, int nrhs, double
     else if (nrhs == 1) shapes = {{256, 0}, {128, 0}, {512, 0}, {256, 1}, {128, 1}};
     if (nrhs == 1) shapes.push_back({SPLIT_SITES, 0});
     const HandSettings unset(c);
-    const double one[2] = {1., 0.};
-    double best         = 1e30;
-    cl2_hop_tuning bt{-1, 1, 1, 1, DSLASH_BLOCK, -1};
+    c->tuned.erase({fmt, nrhs});
+    cl2_hop_tuning usual = hop_tuning(c, fmt, nrhs);
+    usual.rb             = std::max(usual.rb, 1);
+    const double one[2]  = {1., 0.};
+    double best          = 1e30;
+    cl2_hop_tuning bt    = usual;
     int rc = CL2_OK;
     // multi-RHS with one right-hand side per thread: with and without the per-site LDS staging
     std::vector<std::pair<int, int>> rls;
@@ -2001,8 +2004,8 @@ int cl2_autotune_dslash(cl2_ctx* c, const void* gauge, int fmt, int nrhs, double
         ms_out = ms / n;
         return CL2_OK;
     };
-    // every shape briefly; then the three fastest again over four times the launches, so that one short
-    // measurement caught in a clock or power transient does not decide
+    // every shape briefly; then the default and the three fastest again, each the best of three runs of four times the
+    // launches, so that one short measurement caught in a clock or power transient does not decide
     std::vector<std::pair<double, cl2_hop_tuning>> timed;
     for (int zp : zps)
         for (int x : {1, 0})
@@ -2017,14 +2020,17 @@ int cl2_autotune_dslash(cl2_ctx* c, const void* gauge, int fmt, int nrhs, double
     if (rc == CL2_OK) {
         std::stable_sort(timed.begin(), timed.end(),
                          [](const auto& a, const auto& b) { return a.first < b.first; });
-        for (size_t k = 0; k < timed.size() && k < 3 && rc == CL2_OK; ++k) {
-            double ms = 0.;
-            if ((rc = time_shape(timed[k].second, 20, ms)) != CL2_OK) break;
-            if (ms < best) {
-                best = ms;
-                bt   = timed[k].second;
+        std::vector<cl2_hop_tuning> last = {usual};
+        for (size_t k = 0; k < timed.size() && k < 3; ++k) last.push_back(timed[k].second);
+        for (const cl2_hop_tuning& t : last)
+            for (int k = 0; k < 3 && rc == CL2_OK; ++k) {
+                double ms = 0.;
+                if ((rc = time_shape(t, 20, ms)) != CL2_OK) break;
+                if (ms < best) {
+                    best = ms;
+                    bt   = t;
+                }
             }
-        }
     }
     if (rc) {
         c->tuned.erase({fmt, nrhs});
