@@ -403,8 +403,8 @@ hipError_t launch_block_reduce2(cl2_ctx* c, const double2* parts, unsigned nb, d
     };
     // Many partials: 512 threads with four loads in flight (7.4 us for the 20736 per right-hand side of 16 at 48^3x12;
     // with one load 18.6 for the 41472 that were there before).  1024 with eight hold four times the registers, and on
-    // a device that other contexts keep busy such a block waits for a compute unit to come free: two CG steps on 12 FP16
-    // right-hand sides at 30^3x22 took 2309 us with one load in flight, 2367 with those, 2297 with these (alone on the
+    // a device that other contexts keep busy such a block waits for a compute unit to come free: two CG steps on 12
+    // FP16 right-hand sides at 30^3x22 took 2309 us with one load in flight, 2367 with those, 2297 with these (alone on the
     // device 2222, 2187, 2184); four on 4 staggered ones at 32^3x32 918, 942, 912 (1097, 1075, 1076)
     if (nb >= WIDE_SUM_MIN)
         tail ? go(k_block_reduce2<512, 4, true>, 512, *tail) : go(k_block_reduce2<512, 4, false>, 512, NoTail{});
