@@ -743,8 +743,8 @@ __global__ __launch_bounds__(BLOCK) void k_sitediag(vec2<R>* __restrict__ out, c
  * itself, and (in brackets) with three contexts at work, which fill it.  There its half spinors in LDS count from
  * about 28,000 FP64 or 50,000 FP32 and FP16 sites on.  Thread per site / wave per hop in us, QplusQminus_eo of four
  * hopping terms, both in site order; FP16: a pass of four CG steps:
- *   F64_18  8^4 37.3 / 19.9 (18.1 / 15.2), 12^3x20 51.4 / 38.7 (23.9 / 22.4), 14^3x20 57.8 / 46.4 (31.5 / 33.0; 33.2
- *           before either kernel's present order), but 14^3x26 59.4 / 60.9 (40.8 / 42.5), 16^3x24 63.5 / 72.3
+ *   F64_18  8^4 37.3 / 19.9 (18.1 / 15.2), 12^3x20 51.4 / 38.7 (23.9 / 22.4), 14^3x20 57.8 / 46.4 (31.5 / 33.0), but
+ *           14^3x26 59.4 / 60.9 (40.8 / 42.5), 16^3x24 63.5 / 72.3 (54.8 / 54.9)
  *   F64_12  8^4 32.6 / 18.6 (16.0 / 15.2), 12^3x20 42.8 / 31.3 (19.1 / 17.9), 12^3x28 45.3 / 34.4 (24.3 / 24.7), but
  *           14^3x22 48.7 / 38.8 (28.0 / 29.5), 14^3x26 49.1 / 50.7 (32.5 / 33.9)
  *   F32     8^4 24.4 / 15.0 (15.5 / 15.5), 14^3x22 33.0 / 23.0 (19.6 / 18.2), 16^3x24 34.8 / 31.2 (23.6 / 23.9), but
